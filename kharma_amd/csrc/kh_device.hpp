@@ -25,6 +25,12 @@ template <typename R> struct FourVec { R ucon[4], ucov[4], bcon[4], bcov[4]; };
 template <typename R> __device__ __forceinline__ R dot4(const R a[4], const R b[4]) {
     return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
 }
+// b^mu b_mu.  In curved space the second product is the one rounded on its own (see
+// CachedGeom::sum_b).
+template <class G, typename R> __device__ __forceinline__ R bsq_of(const R b[4], const R c[4]) {
+    if constexpr (G::flat) return dot4(b, c);
+    else return fma(b[3], c[3], fma(b[2], c[2], fma(b[0], c[0], b[1] * c[1])));
+}
 template <typename R> __device__ __forceinline__ R dmax(R a, R b) { return a > b ? a : (b != b ? b : a); }
 // std::max / std::min semantics (return the first argument unless the second compares greater/less)
 template <typename R> __device__ __forceinline__ R smax(R a, R b) { return (a < b) ? b : a; }
@@ -90,8 +96,15 @@ template <typename R, bool A32 = false> struct CachedGeom {
     const R* __restrict__ p;
     long np, q;
     __device__ __forceinline__ CachedGeom(const R* __restrict__ base, long np_, long q_) : p(base), np(np_), q(q_) {}
+    // Index of component (a, b) in the packed upper triangle.  Written without
+    // recursion: as sym(b, a) for a > b it was not folded after unrolling, and every
+    // transposed component cost a scalar loop, a 64-bit multiply and a load of its
+    // own (12 of the 32 metric loads of the pair of lower()s in calc_4vecs).  Folded,
+    // both orders share one load: FP64 X2 faces of the 192x128x128 torus 275 -> 234
+    // us, X1 230 -> 192 us, recovery 228 -> 209 us.
     static __device__ __forceinline__ constexpr int sym(int a, int b) {
-        return (a <= b) ? (a == 0 ? b : a == 1 ? 3 + b : a == 2 ? 5 + b : 9) : sym(b, a);
+        const int l = a < b ? a : b, h = a < b ? b : a;
+        return l == 0 ? h : l == 1 ? 3 + h : l == 2 ? 5 + h : 9;
     }
     __device__ __forceinline__ R comp(int n) const {
         if constexpr (A32) return at32(p, (unsigned)(n * np + q));
@@ -102,15 +115,31 @@ template <typename R, bool A32 = false> struct CachedGeom {
     __device__ __forceinline__ R gcon0(int v) const { return gcon(0, v); }
     __device__ __forceinline__ R gdet() const { return comp(20); }
     __device__ __forceinline__ R alpha() const { return comp(21); }
+    // Sums over an index run from 0 to 3.  Which product of the first pair is rounded
+    // before the fused additions start is written out (the second in sum_b, the first
+    // in sum_a) rather than left to the compiler's contraction, which chooses by the
+    // shape of the surrounding code: a step's bits then do not move when a kernel is
+    // arranged differently.
+    static __device__ __forceinline__ R sum_b(R a, R x, R b, R y, R c, R z, R d, R w) {
+        return fma(d, w, fma(c, z, fma(a, x, b * y)));
+    }
+    static __device__ __forceinline__ R sum_a(R a, R x, R b, R y, R c, R z, R d, R w) {
+        return fma(d, w, fma(c, z, fma(b, y, a * x)));
+    }
     __device__ __forceinline__ void lower(const R v[4], R o[4]) const {
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-            o[m] = gcov(m, 0) * v[0] + gcov(m, 1) * v[1] + gcov(m, 2) * v[2] + gcov(m, 3) * v[3];
+        o[0] = sum_b(gcov(0, 0), v[0], gcov(0, 1), v[1], gcov(0, 2), v[2], gcov(0, 3), v[3]);
+        o[1] = sum_a(gcov(1, 0), v[0], gcov(1, 1), v[1], gcov(1, 2), v[2], gcov(1, 3), v[3]);
+        o[2] = sum_b(gcov(2, 0), v[0], gcov(2, 1), v[1], gcov(2, 2), v[2], gcov(2, 3), v[3]);
+        o[3] = sum_b(gcov(3, 0), v[0], gcov(3, 1), v[1], gcov(3, 2), v[2], gcov(3, 3), v[3]);
+    }
+    // o[0] of lower() with its first product rounded first (the recovery's u_t).
+    __device__ __forceinline__ R lower0_a(const R v[4]) const {
+        return sum_a(gcov(0, 0), v[0], gcov(0, 1), v[1], gcov(0, 2), v[2], gcov(0, 3), v[3]);
     }
     __device__ __forceinline__ void raise(const R v[4], R o[4]) const {
 #pragma unroll
         for (int m = 0; m < 4; ++m)
-            o[m] = gcon(m, 0) * v[0] + gcon(m, 1) * v[1] + gcon(m, 2) * v[2] + gcon(m, 3) * v[3];
+            o[m] = sum_b(gcon(m, 0), v[0], gcon(m, 1), v[1], gcon(m, 2), v[2], gcon(m, 3), v[3]);
     }
     // GRMHD::lorentz_calc, grmhd_functions.hpp:116-129
     __device__ __forceinline__ R lorentz(R u1, R u2, R u3) const {
@@ -288,8 +317,8 @@ __device__ __forceinline__ void face_states(const R x[6], R& ql, R& qr) {
 }
 
 // ----------------------------------------------------------------- GRMHD
-// GRMHD::calc_4vecs, grmhd/grmhd_functions.hpp:225-246
-template <typename R, class G>
+// GRMHD::calc_4vecs, grmhd/grmhd_functions.hpp:225-246.  U0A: u_t by lower0_a.
+template <typename R, bool U0A = false, class G>
 __device__ __forceinline__ void calc_4vecs(const G& g, const R P[NV], FourVec<R>& D) {
     const R gamma = g.lorentz(P[U1], P[U2], P[U3]);
     if constexpr (G::flat) {
@@ -301,6 +330,7 @@ __device__ __forceinline__ void calc_4vecs(const G& g, const R P[NV], FourVec<R>
         for (int v = 0; v < 3; ++v) D.ucon[v + 1] = P[U1 + v] - gamma * alpha * g.gcon0(v + 1);
     }
     g.lower(D.ucon, D.ucov);
+    if constexpr (U0A) D.ucov[0] = g.lower0_a(D.ucon);
     D.bcon[0] = P[B1] * D.ucov[1] + P[B2] * D.ucov[2] + P[B3] * D.ucov[3];
     const R iu0 = rcp(D.ucon[0]);
     for (int v = 0; v < 3; ++v) D.bcon[v + 1] = (P[B1 + v] + D.bcon[0] * D.ucon[v + 1]) * iu0;
@@ -313,7 +343,7 @@ template <typename R, class G, int DIR>
 __device__ __forceinline__ void prim_to_u_and_flux(const G& g, const R P[NV], const FourVec<R>& D, R gam,
                                                    R U[NV], R F[NV]) {
     const R gdet = g.gdet();
-    const R bsq = dot4(D.bcon, D.bcov);
+    const R bsq = bsq_of<G>(D.bcon, D.bcov);
     const R pgas = (gam - R(1)) * P[UU];
     const R eta = pgas + P[RHO] + P[UU] + bsq;
     const R ptot = pgas + R(0.5) * bsq;
@@ -349,7 +379,7 @@ template <typename R, class G, int DIR>
 __device__ __forceinline__ void vchar(const G& g, const R P[NV], const FourVec<R>& D, R gam, R& cmax, R& cmin) {
     const R ef = P[RHO] + gam * P[UU];
     const R cs2 = gam * (gam - R(1)) * P[UU] * rcp(ef);
-    const R bsq = dot4(D.bcon, D.bcov);
+    const R bsq = bsq_of<G>(D.bcon, D.bcov);
     const R va2 = bsq * rcp(bsq + ef);
     const R cms2 = cs2 + va2 - cs2 * va2;
     R A, B, C;

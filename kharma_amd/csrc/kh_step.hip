@@ -141,7 +141,7 @@ __device__ __forceinline__ void add_geo_source_c(const G& g, const C& conn, cons
                                                  double dudt[NV]) {
     FourVec<double> D;
     calc_4vecs<double>(g, Psub, D);
-    const double bsq = dot4(D.bcon, D.bcov);
+    const double bsq = bsq_of<G>(D.bcon, D.bcov);
     const double pgas = (gam - 1.) * Psub[UU];
     const double eta = pgas + Psub[RHO] + Psub[UU] + bsq;
     const double ptot = pgas + 0.5 * bsq;
@@ -710,7 +710,7 @@ __device__ __forceinline__ void recover_zone(const BlockDims& b, const StepConst
         const double igd = rcp(gd_);
         P[B1] = U[B1] * igd; P[B2] = U[B2] * igd; P[B3] = U[B3] * igd;
         FourVec<double> D;
-        calc_4vecs<double>(g, P, D);
+        calc_4vecs<double, true>(g, P, D);
         ff = ff0;
         if (cst.floors.on) ff = floors_zone<FRAME>(g, P, U, D, gam, cst.floors, rf, uf, ff0, pf);
         p_to_u_D(g, P, D, gam, U);
