@@ -181,19 +181,16 @@ flux_x1_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> 
 
 // X2 / X3 faces.  Transverse columns: flattened (outer, i) with i in [is-1, ie+1]
 // fastest; outer = k (X2) or j (X3) from o0.  Along the normal: faces s in
-// [s0, s1]; tile y covers cells s0-1+(TY-1)y .. s0-2+TY+(TY-1)y.  TY matches the
-// block to the waves a CU holds at the variant's registers: the curved-space
-// FP64 variant (~142 VGPRs, 3 waves per SIMD) runs 64 x 12 blocks, one per CU at
-// 12 waves (5 % faster than 64 x 8, whose one block per CU holds 8); the others
-// (FP32 ~92, flat FP64 ~104 VGPRs) run 64 x 8, two blocks per CU (64 x 10 and
-// 64 x 16 FP32 blocks measured 24 % and 2 % slower).
-template <typename R, int GEO> struct XtTile { static constexpr int TY = (sizeof(R) == 8 && GEO) ? 12 : 8; };
+// [s0, s1]; tile y covers cells s0-1+(TY-1)y .. s0-2+TY+(TY-1)y.  64 x 8 blocks, two (FP64, 103-118 VGPRs)
+// or three (FP32, 63) per CU: 64 x 10 and 64 x 16 FP32 blocks measured 24 % and 2 %
+// slower, 64 x 4, 64 x 12 and 64 x 16 FP64 blocks 5, 3 and 4 % (192x128x128 torus).
+constexpr int XT_TY = 8;
 template <int DIR, int RECON, int SPEEDS, typename R, typename PT, int GEO, bool PK>
-__global__ void __launch_bounds__((64 * XtTile<R, GEO>::TY), XtOcc<R>::w)
+__global__ void __launch_bounds__(64 * XT_TY, XtOcc<R>::w)
 flux_xt_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> F,
                R* __restrict__ cmax_out, R* __restrict__ cmin_out, int o0, int no, int s0, int s1,
                const BlockEntry* __restrict__ pk) {
-    constexpr int TY = XtTile<R, GEO>::TY;
+    constexpr int TY = XT_TY;
     __shared__ R sr[NV][TY][64];
     if constexpr (PK) {
         const long blk = pack_select(pk, b, gd);
@@ -242,6 +239,292 @@ flux_xt_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> 
     face_flux<DIR, SPEEDS, R, GEO>(c, b, gd, jf, if_, Pl, lo, ci, F, cmax_out, cmin_out);
 }
 
+// ---------------------------------------------------- FP64, large 3-D blocks
+// The tile kernels keep four (FP64) wavefronts per SIMD waiting half their life:
+// 40 stencil loads, a barrier, the metric's loads, all in one short pass per face.
+// The marching kernels walk instead.
+//
+// X2 / X3 faces.  Each lane walks its own column of cells
+// along the face normal, over a chunk of faces, with the five cells of the stencil
+// in registers, so a row costs 8 loads of P instead of 40 and each cell is
+// reconstructed once.
+//
+// Nothing in a row waits for memory: the cell that enters the next row's stencil
+// and (X2) the next row's metric are requested at the row's start and used a row
+// later, and no other load follows them (loads complete in order, so any later one
+// would wait for both).  The metric of the row sits in the lane's own LDS slots,
+// as do the two face states, which frees the registers the window needs (two
+// waves per SIMD).  Lanes share nothing: there is no barrier.
+//
+// Bound by FP64 issue and its dependent chains: VALU 68 % busy at two wavefronts
+// (45 % for the tiles at three), 24 % fewer instructions a face.  192x128x128 torus:
+// X2 234 -> 165 us, X3 226 -> 144 us.  Asking for the next row before the metric
+// (249 us X2: the metric's waits included the prefetch) and the metric straight
+// from memory behind it (250 us X2, 182 us X3) were slower.
+//
+// LaneGeom: one lane's metric in LDS, components the flux needs, [MG_N][256].
+enum { MG_G00, MG_G01, MG_G03, MG_G11, MG_G12, MG_G13, MG_G22, MG_G33, MG_U00, MG_U01, MG_U02, MG_U03, MG_UDD, MG_GDET, MG_ALPHA, MG_RF, MG_UF, MG_N };
+template <int RECON>
+__device__ __forceinline__ void march_states(double x1, double x2, double x3, double x4, double x5, double& lout, double& rout) {
+    if constexpr (RECON == RECON_WENO5) weno5_cell_lean(x1, x2, x3, x4, x5, lout, rout);
+    else cell_states<RECON, double>(x1, x2, x3, x4, x5, lout, rout);
+}
+template <int DIR> struct LaneGeom {
+    static constexpr bool flat = false;
+    const double (*s)[256];
+    int t;
+    static __device__ __forceinline__ constexpr int src(int m) {   // component of the cached table
+        return m == MG_G00 ? 0 : m == MG_G01 ? 1 : m == MG_G03 ? 3 : m == MG_G11 ? 4 : m == MG_G12 ? 5 : m == MG_G13 ? 6
+             : m == MG_G22 ? 7 : m == MG_G33 ? 9 : m == MG_U00 ? 10 : m == MG_U01 ? 11 : m == MG_U02 ? 12 : m == MG_U03 ? 13
+             : m == MG_UDD ? (DIR == 1 ? 14 : DIR == 2 ? 17 : 19) : m == MG_GDET ? GEO_GDET : GEO_ALPHA;
+    }
+    __device__ __forceinline__ double gcov(int a, int b) const {
+        const int l = a < b ? a : b, h = a < b ? b : a;
+        return s[l == 0 ? (h == 0 ? MG_G00 : h == 1 ? MG_G01 : MG_G03)
+               : l == 1 ? (h == 1 ? MG_G11 : h == 2 ? MG_G12 : MG_G13) : l == 2 ? MG_G22 : MG_G33][t];
+    }
+    __device__ __forceinline__ double gcon(int a, int b) const {
+        return a == 0 ? s[MG_U00 + b][t] : s[MG_UDD][t];
+    }
+    __device__ __forceinline__ double gcon0(int v) const { return s[MG_U00 + v][t]; }
+    __device__ __forceinline__ double gdet() const { return s[MG_GDET][t]; }
+    __device__ __forceinline__ double alpha() const { return s[MG_ALPHA][t]; }
+    // CachedGeom::lower without the products with g_{t x2} and g_{x2 phi}, which vanish
+    __device__ __forceinline__ void lower(const double v[4], double o[4]) const {
+        o[0] = fma(gcov(0, 3), v[3], fma(gcov(0, 0), v[0], gcov(0, 1) * v[1]));
+        o[1] = sum_a(gcov(0, 1), v[0], gcov(1, 1), v[1], gcov(1, 2), v[2], gcov(1, 3), v[3]);
+        o[2] = fma(gcov(2, 2), v[2], gcov(1, 2) * v[1]);
+        o[3] = fma(gcov(3, 3), v[3], fma(gcov(0, 3), v[0], gcov(1, 3) * v[1]));
+    }
+    __device__ __forceinline__ double lorentz(double u1, double u2, double u3) const {
+        const double qsq = gcov(1, 1) * u1 * u1 + gcov(2, 2) * u2 * u2 + gcov(3, 3) * u3 * u3 +
+                           2. * (gcov(1, 2) * u1 * u2 + gcov(1, 3) * u1 * u3);
+        return sqrt(1. + qsq);
+    }
+};
+template <int DIR, int RECON, int SPEEDS, int GEO, bool PK>
+__global__ void __launch_bounds__(256, 2)
+flux_march_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const double> P, Vars<double> F,
+                  double* __restrict__ cmax_out, double* __restrict__ cmin_out, int o0, int no, int s0, int s1, int chunk,
+                  const BlockEntry* __restrict__ pk) {
+    if constexpr (PK) {
+        const long blk = pack_select(pk, b, gd);
+        P = pack_at(P, blk * NV * b.nc);
+        F = pack_at(F, blk * 3 * NV * b.nc);
+        cmax_out = pack_at(cmax_out, blk * 3 * b.nc);
+        cmin_out = pack_at(cmin_out, blk * 3 * b.nc);
+    }
+    __shared__ double sl[NV][256], sr[NV][256], sm[GEO ? MG_N : 1][256];
+    const int tid = threadIdx.x;
+    const int ni = b.nx1 + 2;
+    const unsigned col = blockIdx.x * 256u + threadIdx.x;
+    if (col >= (unsigned)ni * (unsigned)no) return;
+    const int outer = o0 + (int)(col / (unsigned)ni);
+    const int i = b.is - 1 + (int)(col % (unsigned)ni);
+    const int first = s0 + (int)blockIdx.y * chunk;
+    const int last = min(first + chunk - 1, s1);
+    const unsigned st = (unsigned)((DIR == 2) ? b.s2 : b.s3);
+    unsigned ci = (unsigned)((DIR == 2) ? outer * b.s3 : outer * b.s2) + (unsigned)i + (unsigned)(first - 1) * st;
+    // the metric of the row's faces: X2 rows have their own, X3 rows share one
+    unsigned q = (unsigned)((DIR == 2) ? first : outer) * (unsigned)gd.gn1 + (unsigned)i;
+    constexpr int loc = (DIR == 2) ? GLOC_FACE2 : GLOC_CENTER;
+    double mg[GEO ? MG_N : 1];
+    auto load_metric = [&](unsigned at) {
+        if constexpr (GEO) {
+#pragma unroll
+            for (int m = 0; m < MG_RF; ++m) mg[m] = at32(gd.g[loc] + (long)LaneGeom<DIR>::src(m) * gd.np, at);
+            mg[MG_RF] = at32(gd.flr, at);
+            mg[MG_UF] = at32(gd.flr + gd.np, at);
+        }
+    };
+    auto store_metric = [&]() {
+        if constexpr (GEO) {
+#pragma unroll
+            for (int m = 0; m < MG_N; ++m) sm[m][tid] = mg[m];
+        }
+    };
+    double w[NV][5];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+#pragma unroll
+        for (int m = 0; m < 5; ++m) w[v][m] = at32(P[v], ci + (unsigned)(m - 2) * st);
+    }
+    unsigned ahead = ci + 3 * st;
+    double pre[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) pre[v] = at32(P[v], ahead);
+    load_metric(q);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        double lo, hi;
+        march_states<RECON>(w[v][0], w[v][1], w[v][2], w[v][3], w[v][4], lo, hi);
+        sl[v][tid] = hi;
+    }
+    store_metric();
+    for (int s = first; s <= last; ++s) {
+        ci += st;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            w[v][0] = w[v][1]; w[v][1] = w[v][2]; w[v][2] = w[v][3]; w[v][3] = w[v][4];
+            w[v][4] = pre[v];
+        }
+        // (the last row requests its own again rather than past the stencil)
+        if (s < last) {
+            ahead += st;
+            if (DIR == 2) q += (unsigned)gd.gn1;
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) pre[v] = at32(P[v], ahead);
+        if constexpr (DIR == 2) load_metric(q);
+        __builtin_amdgcn_sched_barrier(0);
+        double Pl[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            double lo, hi;
+            march_states<RECON>(w[v][0], w[v][1], w[v][2], w[v][3], w[v][4], lo, hi);
+            sr[v][tid] = lo;
+            Pl[v] = sl[v][tid];
+            sl[v][tid] = hi;
+        }
+        double Pr[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) Pr[v] = sr[v][tid];
+        if constexpr (GEO) {
+            LaneGeom<DIR> g{sm, tid};
+            face_flux_g<DIR, SPEEDS, double>(c, b, g, sm[MG_RF][tid], sm[MG_UF][tid], Pl, Pr, (long)ci, F, cmax_out, cmin_out);
+        } else {
+            MinkowskiGeom<double> g;
+            face_flux_g<DIR, SPEEDS, double>(c, b, g, c.floors.rho_min_const, c.floors.u_min_const, Pl, Pr, (long)ci, F,
+                                             cmax_out, cmin_out);
+        }
+        if constexpr (DIR == 2) store_metric();
+    }
+}
+
+// X1 faces of large 3-D blocks in FP64: each lane walks along x3 with one cell of
+// a row, the rows flattened over (x2, x1) with three cells beyond either end, so
+// a wavefront's 64 cells and two more on each side hold every stencil.  A row's 68
+// cells pass through LDS (one load a cell instead of five, requested a row ahead);
+// the metric, which x3 does not change, is read once.  A wavefront takes 63 faces
+// and shares nothing with the others: the LDS exchange needs no barrier, only that
+// its accesses stay in order.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+template <int RECON, int SPEEDS, bool PK>
+__global__ void __launch_bounds__(256, 2)
+flux_x1_march_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const double> P, Vars<double> F,
+                     double* __restrict__ cmax_out, double* __restrict__ cmin_out, int j0, int nj, int k0, int k1, int chunk,
+                     const BlockEntry* __restrict__ pk) {
+    if constexpr (PK) {
+        const long blk = pack_select(pk, b, gd);
+        P = pack_at(P, blk * NV * b.nc);
+        F = pack_at(F, blk * 3 * NV * b.nc);
+        cmax_out = pack_at(cmax_out, blk * 3 * b.nc);
+        cmin_out = pack_at(cmin_out, blk * 3 * b.nc);
+    }
+    __shared__ double row[NV][4][68], sh[NV][256], sm[MG_N][256];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int L = b.nx1 + 6, total = L * nj;
+    const int g0 = ((int)blockIdx.x * 4 + wv) * 63;   // the wavefront's first cell
+    if (g0 >= total) return;                           // (whole wavefronts)
+    auto offset = [&](int g) {                         // of flattened cell g, clamped into the rows
+        g = min(max(g, 0), total - 1);
+        const int jj = (int)((unsigned)g / (unsigned)L);
+        return (unsigned)((j0 + jj) * b.s2) + (unsigned)(b.is - 3 + (g - jj * L));
+    };
+    const int g = g0 + lane;
+    const int jj = (int)((unsigned)min(g, total - 1) / (unsigned)L), ii = g - jj * L;
+    const bool face = lane > 0 && g < total && ii >= 3 && ii <= b.nx1 + 3;
+    const int first = k0 + (int)blockIdx.y * chunk;
+    const int last = min(first + chunk - 1, k1);
+    const unsigned s3 = (unsigned)b.s3;
+    unsigned ci = offset(g) + (unsigned)first * s3;
+    // lanes 0-3 also fetch the two cells before and after the wavefront's
+    const int hm = lane < 2 ? lane : 64 + lane;
+    const bool halo = lane < 4;
+    unsigned hi_ci = offset(g0 - 2 + hm) + (unsigned)first * s3;
+    {
+        const unsigned q = (unsigned)(j0 + jj) * (unsigned)gd.gn1 + (unsigned)(b.is - 3 + min(ii, L - 1));
+#pragma unroll
+        for (int m = 0; m < MG_RF; ++m) sm[m][tid] = at32(gd.g[GLOC_FACE1] + (long)LaneGeom<1>::src(m) * gd.np, q);
+        sm[MG_RF][tid] = at32(gd.flr, q);
+        sm[MG_UF][tid] = at32(gd.flr + gd.np, q);
+    }
+    double pre[NV], prh[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) pre[v] = at32(P[v], ci);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) prh[v] = halo ? at32(P[v], hi_ci) : 0.;
+    for (int k = first; k <= last; ++k) {
+        double own[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            own[v] = pre[v];
+            row[v][wv][lane + 2] = pre[v];
+            if (halo) row[v][wv][hm] = prh[v];
+        }
+        wave_lds_fence();
+        const unsigned at = ci;
+        if (k < last) { ci += s3; hi_ci += s3; }   // (the last row requests its own again)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) pre[v] = at32(P[v], ci);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) prh[v] = halo ? at32(P[v], hi_ci) : 0.;
+        __builtin_amdgcn_sched_barrier(0);
+        double lo[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            double hi;
+            const double* r = &row[v][wv][lane];
+            march_states<RECON>(r[0], r[1], own[v], r[3], r[4], lo[v], hi);
+            sh[v][tid] = hi;
+        }
+        wave_lds_fence();
+        double Pl[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) Pl[v] = sh[v][lane > 0 ? tid - 1 : tid];
+        wave_lds_fence();   // the next row overwrites row and sh
+        if (face) {
+            LaneGeom<1> gm{sm, tid};
+            face_flux_g<1, SPEEDS, double>(c, b, gm, sm[MG_RF][tid], sm[MG_UF][tid], Pl, lo, (long)at, F, cmax_out, cmin_out);
+        }
+    }
+}
+
+// Rows per resident lane from which the marching kernels are used: two wavefronts
+// per SIMD, 131072 lanes.  A walk pays its start (five rows of loads, one extra
+// reconstruction) once per chunk, and two wavefronts hide less latency than the
+// tiles' four, so short walks lose.  Measured, tiles against marching, us: X2/X3
+// 64^3 flat 22 / 25, 99x66x50 torus 32 / 33, 126x90x61 torus 57 / 51, 96^3 flat 64 / 56,
+// 128^3 flat 140 / 111, 192x128x128 torus 246 / 184 and 235 / 163; X1 126x90x61 torus
+// 49 / 52, 192x96x64 81 / 79, 150x110x100 111 / 105, 192x128x128 210 / 180; X1 flat 128^3
+// 112 / 118 (four wavefronts of 103 registers: the tiles stay).  (2-D blocks have one
+// row of each along x3 and too few faces: tiles.)
+constexpr long MARCH_LANES = 2L * 4 * 256 * 64;
+static bool march_xt(const BlockDims& b, long cols, int nfaces, int nblk) {
+    return b.ndim == 3 && cols * nfaces * nblk >= 4 * MARCH_LANES;
+}
+static bool march_x1(const BlockDims& b, long cells, int nblk) {
+    return b.geo && b.ndim == 3 && cells * nblk >= 8 * MARCH_LANES;
+}
+// Faces per chunk: the fewest rounds of work for the busiest CU, a round being one
+// block's chunk plus its start (0.6 of a row's work); a CU holds two blocks, and
+// one alone on it runs at 0.6 of their rate.
+static int march_chunk(long blocks_x, int nfaces) {
+    int best = nfaces;
+    double cost = 1e300;
+    for (int ch = 1; ch <= nfaces; ++ch) {
+        const long blocks = blocks_x * ((nfaces + ch - 1) / ch);
+        const double per_cu = (double)((blocks + 255) / 256);
+        const double t = (per_cu > 1.6 ? per_cu : 1.6) * (ch + 0.6);
+        if (t < cost) { cost = t; best = ch; }
+    }
+    return best;
+}
+
 template <int RECON, int SPEEDS, typename R, typename PT, int GEO, bool PK>
 static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, const Vars<const PT>& P, const Vars<R>& F,
                                R* cmax, R* cmin, hipStream_t s, const Pack* pk) {
@@ -250,6 +533,35 @@ static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const Ge
     // covers [start, end+1]; transverse indices extend one zone each side.
     const int jlo = (b.ndim > 1) ? b.js - 1 : b.js, jhi = (b.ndim > 1) ? b.je + 1 : b.je;
     const int klo = (b.ndim > 2) ? b.ks - 1 : b.ks, khi = (b.ndim > 2) ? b.ke + 1 : b.ke;
+    const int nblk = pk ? pk->nblk : 1;
+    if constexpr (sizeof(R) == 8) {
+        if (dir == 1) {
+            const int nj = jhi - jlo + 1, nk = khi - klo + 1;
+            const long cells = (long)(b.nx1 + 6) * nj;
+            if (march_x1(b, cells * nk, nblk)) {
+                const unsigned bx = (unsigned)((cells + 4 * 63 - 1) / (4 * 63));
+                const int chunk = march_chunk((long)bx * nblk, nk);
+                const dim3 grid = pack_grid(dim3(bx, (unsigned)((nk + chunk - 1) / chunk)), pk);
+                hipLaunchKernelGGL((flux_x1_march_kernel<RECON, SPEEDS, PK>), grid, dim3(256), 0, s, b, c, gd, P, F, cmax, cmin, jlo, nj, klo, khi, chunk, pd);
+                return hipGetLastError();
+            }
+        } else {
+            const int o0 = dir == 2 ? klo : jlo, no = dir == 2 ? khi - klo + 1 : jhi - jlo + 1;
+            const int s0 = dir == 2 ? b.js : b.ks, s1 = dir == 2 ? b.je + 1 : b.ke + 1;
+            const long cols = (long)(b.nx1 + 2) * no;
+            const int nfaces = s1 - s0 + 1;
+            if (march_xt(b, cols, nfaces, nblk)) {
+                const unsigned bx = (unsigned)((cols + 255) / 256);
+                const int chunk = march_chunk((long)bx * nblk, nfaces);
+                const dim3 grid = pack_grid(dim3(bx, (unsigned)((nfaces + chunk - 1) / chunk)), pk);
+                if (dir == 2)
+                    hipLaunchKernelGGL((flux_march_kernel<2, RECON, SPEEDS, GEO, PK>), grid, dim3(256), 0, s, b, c, gd, P, F, cmax, cmin, o0, no, s0, s1, chunk, pd);
+                else
+                    hipLaunchKernelGGL((flux_march_kernel<3, RECON, SPEEDS, GEO, PK>), grid, dim3(256), 0, s, b, c, gd, P, F, cmax, cmin, o0, no, s0, s1, chunk, pd);
+                return hipGetLastError();
+            }
+        }
+    }
     if (dir == 1) {
         const int nj = jhi - jlo + 1, nk = khi - klo + 1;
         const long cells = (long)(b.nx1 + 2) * nj * nk;
@@ -259,14 +571,14 @@ static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const Ge
         const int no = khi - klo + 1;
         const int ncol = (b.nx1 + 2) * no;
         const int nfaces = b.nx2 + 1;
-        constexpr int TY = XtTile<R, GEO>::TY;
+        constexpr int TY = XT_TY;
         const dim3 grid = pack_grid(dim3((unsigned)((ncol + 63) / 64), (unsigned)((nfaces + TY - 2) / (TY - 1))), pk);
         hipLaunchKernelGGL((flux_xt_kernel<2, RECON, SPEEDS, R, PT, GEO, PK>), grid, dim3(64, TY), 0, s, b, c, gd, P, F, cmax, cmin, klo, no, b.js, b.je + 1, pd);
     } else {
         const int no = jhi - jlo + 1;
         const int ncol = (b.nx1 + 2) * no;
         const int nfaces = b.nx3 + 1;
-        constexpr int TY = XtTile<R, GEO>::TY;
+        constexpr int TY = XT_TY;
         const dim3 grid = pack_grid(dim3((unsigned)((ncol + 63) / 64), (unsigned)((nfaces + TY - 2) / (TY - 1))), pk);
         hipLaunchKernelGGL((flux_xt_kernel<3, RECON, SPEEDS, R, PT, GEO, PK>), grid, dim3(64, TY), 0, s, b, c, gd, P, F, cmax, cmin, jlo, no, b.ks, b.ke + 1, pd);
     }
