@@ -61,7 +61,7 @@ namespace {
     } while (0)
 
 // One forward stage on the driver's buffers, as kh::driver_stage runs it,
-// keeping U* (between the update's combine and recovery halves), the floor
+// keeping U* (as the update's recovery finds it), the floor
 // flags and the clamped X1 mass fluxes of the stage.
 int recompute_stage(kh_adjoint* a, int stage) {
     kh_driver* d = a->drv;
@@ -86,8 +86,8 @@ int recompute_stage(kh_adjoint* a, int stage) {
         KA_HIP(launch_save_x1_flux(bd, F, a->x1f[stage - 1], s));
     }
     if (a->geo) {
-        KA_HIP(launch_update_parts(bd, c, b->geo, stage, 3, F, Usub, d->U0, Psub, Uout, Pout, pflag, fflag,
-                                   d->fail_list, d->ds, s, a->Ustar[stage - 1]));
+        KA_HIP(launch_update_recorded(bd, c, b->geo, stage, false, F, ct, Usub, d->U0, Psub, Uout, Pout, pflag,
+                                      fflag, d->fail_list, d->ds, d->dt_part, a->Ustar[stage - 1], s));
     } else {
         KA_HIP(launch_update(bd, c, b->geo, b->p.precision, stage, false, F, ct, Usub, d->U0, Psub, Uout, Pout,
                              nullptr, pflag, fflag, d->fail_list, d->ds, d->dt_part, s));

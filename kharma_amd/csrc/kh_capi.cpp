@@ -827,7 +827,7 @@ int kh_driver_create(const kh_params* p, kh_driver** out) {
         if ((e = hipMalloc(&d->P0f, sizeof(float) * NV * nc)) != hipSuccess) return cleanup(e, "hipMalloc P0f");
         if ((e = hipMalloc(&d->P1f, sizeof(float) * NV * nc)) != hipSuccess) return cleanup(e, "hipMalloc P1f");
     }
-    if ((e = hipMalloc(&d->dt_part, sizeof(double) * (update_blocks(blk->dims) + 1))) != hipSuccess) return cleanup(e, "hipMalloc dt_part");
+    if ((e = hipMalloc(&d->dt_part, sizeof(double) * (dt_blocks(blk->dims) + 1))) != hipSuccess) return cleanup(e, "hipMalloc dt_part");
     if ((e = hipMalloc(&d->divb_part, sizeof(double) * (divb_blocks(blk->dims) + 1))) != hipSuccess) return cleanup(e, "hipMalloc divb_part");
     if ((e = hipMalloc(&d->pflag, sizeof(int) * nc)) != hipSuccess) return cleanup(e, "hipMalloc pflag");
     if ((e = hipMalloc(&d->fflag, sizeof(int) * nc)) != hipSuccess) return cleanup(e, "hipMalloc fflag");
@@ -1059,7 +1059,7 @@ int kh_driver_step(kh_driver* d, int nsteps) {
     const BlockDims& bd = b->dims;
     const StepConsts& c = b->consts;
     hipStream_t s = b->stream;
-    const int n_dt = (int)update_blocks(bd), n_divb = (int)divb_blocks(bd);
+    const int n_dt = (int)dt_blocks(bd), n_divb = (int)divb_blocks(bd);
     for (int n = 0; n < nsteps; ++n) {
         for (int stage = 1; stage <= 2; ++stage) {
             const int st = driver_stage(d, stage);

@@ -241,7 +241,7 @@ int kh_mesh_create(const kh_params* p, int nb1, int nb2, int nb3, kh_mesh** out)
             k->geo = m->blk[b % (nb1 * nb2)]->geo;
         }
     const BlockDims& bd = m->blk[0]->dims;
-    m->n_dt = update_blocks(bd);
+    m->n_dt = dt_blocks(bd);
     m->n_divb = divb_blocks(bd);
     const long nc = md.nc, nblk = md.nblk;
     const size_t sb = sizeof(double) * NV * nc * nblk;

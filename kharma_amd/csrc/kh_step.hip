@@ -1,180 +1,16 @@
-// kh_step.hip -- flux-CT, the fused stage update, inversion fix-ups, reductions
-// and the task-level kernels that mirror the reference's individual tasks.
-//
-// The fused update kernel performs, for one interior zone and in registers:
-//   flux-CT B fluxes from the corner EMFs (B_FluxCT::FluxCT, b_flux_ct.cpp:347-369)
-//   + flux divergence (KHARMADriver::FluxDivergence, kharma_driver.hpp:208-231)
-//   + RK state update (KHARMADriver::AddStateUpdate, kharma_driver.cpp:339-387)
-//   + onedw U->P (Inverter::BlockUtoP, inverter.cpp:131-182) and B U->P (b_flux_ct.cpp:195-217)
-//   + floors (Floors::ApplyGRMHDFloors, floors_impl.hpp:45-128)
-//   + P->U (Flux::MeshPtoU, flux.cpp:276-322)
-//   + (last stage) the CFL estimate (GRMHD::EstimateTimestep, grmhd.cpp:313-328)
-// and writes U, P and the flags once, also into the periodic ghost images of
-// the zone (the boundary exchange), so no separate sync pass reads the state.
+// kh_step.hip -- flux-CT, inversion fix-ups, reductions and the task-level kernels
+// that mirror the reference's individual tasks.
 #include <algorithm>
 #include <mutex>
 
-#include "kh_internal.hpp"
-
-#include <cfloat>
+#include "kh_step.hpp"
 
 namespace kh {
-
-static constexpr int BS = 256;
-// Work-groups per CU the update kernel is compiled for: 4 (128 VGPRs) with the
-// flat metric; the cached-metric variant needs ~240 VGPRs and would spill at 4.
-template <int GEO> struct UpdateOcc { static constexpr int min_blocks = GEO ? 2 : 4; };
-
-static inline dim3 grid_for(long n, int bs = BS) { return dim3((unsigned)((n + bs - 1) / bs)); }
-static inline long ninterior_host(const BlockDims& b) {
-    return (long)b.nx1 * (b.ndim > 1 ? b.nx2 : 1) * (b.ndim > 2 ? b.nx3 : 1);
-}
 
 // FP32 shadow of the primitives read by the split-precision flux kernels.
 __global__ void __launch_bounds__(256) convert_f32_kernel(const double* __restrict__ A, float* __restrict__ B, long n) {
     const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t < n) B[t] = (float)A[t];
-}
-
-// ------------------------------------------------------------ ghost images
-// Images of interior zone (k,j,i) in ghost regions: per axis, the zone's
-// offset in the image block's layout (0 = no image) and the index offset of
-// that block (0: this block, a periodic axis of a one-block mesh; otherwise
-// the neighbour across the face the zone lies within ng of).  With nx >= 2 ng
-// on every image axis a zone has at most one image per axis, so up to 7 image
-// copies (edges and corners land in the diagonal neighbour, whose block offset
-// is the sum of the axes' offsets).
-struct ImageSet {
-    long oi, oj, ok;
-    int bi, bj, bk;
-};
-__device__ __forceinline__ void image_set(const BlockDims& b, int k, int j, int i, ImageSet& s) {
-    s.oi = s.oj = s.ok = 0;
-    s.bi = s.bj = s.bk = 0;
-    if (b.img[0][0] && i - b.is < b.ng) { s.oi = b.nx1; s.bi = b.nbd[0][0]; }
-    else if (b.img[0][1] && b.ie - i < b.ng) { s.oi = -b.nx1; s.bi = b.nbd[0][1]; }
-    if (b.ndim > 1) {
-        if (b.img[1][0] && j - b.js < b.ng) { s.oj = (long)b.nx2 * b.s2; s.bj = b.nbd[1][0]; }
-        else if (b.img[1][1] && b.je - j < b.ng) { s.oj = -(long)b.nx2 * b.s2; s.bj = b.nbd[1][1]; }
-    }
-    if (b.ndim > 2) {
-        if (b.img[2][0] && k - b.ks < b.ng) { s.ok = (long)b.nx3 * b.s3; s.bk = b.nbd[2][0]; }
-        else if (b.img[2][1] && b.ke - k < b.ng) { s.ok = -(long)b.nx3 * b.s3; s.bk = b.nbd[2][1]; }
-    }
-}
-// base[c] = val and the same at every image; bstride: elements between the
-// same array of consecutive blocks (NV nc for a state, nc for a flag array).
-template <typename T>
-__device__ __forceinline__ void store_with_images(const BlockDims&, const ImageSet& s, T* base, long c, T val,
-                                                  long bstride) {
-    base[c] = val;
-    if ((s.oi | s.oj | s.ok) == 0) return;
-    const long di = s.oi + s.bi * bstride, dj = s.oj + s.bj * bstride, dk = s.ok + s.bk * bstride;
-    if (s.oi) base[c + di] = val;
-    if (s.oj) base[c + dj] = val;
-    if (s.ok) base[c + dk] = val;
-    if (s.oi && s.oj) base[c + di + dj] = val;
-    if (s.oi && s.ok) base[c + di + dk] = val;
-    if (s.oj && s.ok) base[c + dj + dk] = val;
-    if (s.oi && s.oj && s.ok) base[c + di + dj + dk] = val;
-}
-
-__device__ __forceinline__ void interior_index(const BlockDims& b, unsigned t, int& k, int& j, int& i) {
-    const unsigned nij = (unsigned)b.nx1 * (unsigned)(b.ndim > 1 ? b.nx2 : 1);
-    const unsigned kk = t / nij;
-    const unsigned rem = t - kk * nij;
-    const unsigned jj = rem / (unsigned)b.nx1;
-    i = b.is + (int)(rem - jj * (unsigned)b.nx1);
-    j = b.js + (int)jj;
-    k = b.ks + (int)kk;
-}
-__device__ __forceinline__ long ninterior(const BlockDims& b) {
-    return (long)b.nx1 * (b.ndim > 1 ? b.nx2 : 1) * (b.ndim > 2 ? b.nx3 : 1);
-}
-
-// Metric of cell centre (j, i): flat, or read from the geometry cache.
-template <int GEO, class Fn>
-__device__ __forceinline__ void with_center_geom(const GeomDev& gd, int j, int i, Fn&& fn) {
-    if constexpr (GEO) {
-        CachedGeom<double> g(gd.g[GLOC_CENTER], gd.np, (long)j * gd.gn1 + i);
-        fn(g);
-    } else {
-        MinkowskiGeom<double> g;
-        fn(g);
-    }
-}
-// Geometric floors of cell centre (j, i) (floors_functions.hpp:97-108)
-template <int GEO>
-__device__ __forceinline__ void geom_floors(const StepConsts& c, const GeomDev& gd, int j, int i, double& rf, double& uf) {
-    if constexpr (GEO) {
-        const long q = (long)j * gd.gn1 + i;
-        rf = gd.flr[q];
-        uf = gd.flr[gd.np + q];
-    } else {
-        rf = c.floors.rho_min_const;
-        uf = c.floors.u_min_const;
-    }
-}
-// KDomain::GetPhysicalRange (domain.hpp:161-187): the entire block, less the
-// ghosts across physical-boundary faces (the ghosts of periodic faces and of
-// faces shared with another block are in range).
-__device__ __forceinline__ bool in_physical(const BlockDims& b, int k, int j, int i) {
-    if (i < 0 || i >= b.n1 || j < 0 || j >= b.n2 || k < 0 || k >= b.n3) return false;
-    if ((i < b.is && !b.img[0][0]) || (i > b.ie && !b.img[0][1])) return false;
-    if (b.ndim > 1 && ((j < b.js && !b.img[1][0]) || (j > b.je && !b.img[1][1]))) return false;
-    if (b.ndim > 2 && ((k < b.ks && !b.img[2][0]) || (k > b.ke && !b.img[2][1]))) return false;
-    return true;
-}
-
-// Flux::AddGeoSource (flux/flux.cpp:395-444): the T^mu_nu Gamma contraction of
-// zone (j, i) added to the energy and momentum rates,
-// S_lam = sum_{mu, nu} T^mu_nu sqrt(-g) Gamma^nu_{lam mu}.  conn holds
-// sqrt(-g) Gamma^a_{b c} at index 16 a + 4 b + c, exactly symmetric in (b, c)
-// (the geometry build stores the mean of the two finite-difference orders), so
-// each of the 40 distinct components is loaded once and serves both (lam, mu)
-// and (mu, lam): 40 loads instead of 64 (the reference sums all 64; the sum
-// here differs from it by rounding only).  No test for zero components: a
-// branch per component would make every load wait for the one before it.
-// conn(n) returns component n = 16 a + 4 b + c of this zone's table.
-template <class G, class C>
-__device__ __forceinline__ void add_geo_source_c(const G& g, const C& conn, const double Psub[NV], double gam,
-                                                 double dudt[NV]) {
-    FourVec<double> D;
-    calc_4vecs<double>(g, Psub, D);
-    const double bsq = bsq_of<G>(D.bcon, D.bcov);
-    const double pgas = (gam - 1.) * Psub[UU];
-    const double eta = pgas + Psub[RHO] + Psub[UU] + bsq;
-    const double ptot = pgas + 0.5 * bsq;
-    double nd[4] = {0., 0., 0., 0.};
-    double T[4][4];   // T^mu_nu
-#pragma unroll
-    for (int mu = 0; mu < 4; ++mu)
-#pragma unroll
-        for (int nu = 0; nu < 4; ++nu) T[mu][nu] = eta * D.ucon[mu] * D.ucov[nu] + (mu == nu ? ptot : 0.) - D.bcon[mu] * D.bcov[nu];
-#pragma unroll
-    for (int nu = 0; nu < 4; ++nu) {
-        double cs[10];
-#pragma unroll
-        for (int lam = 0, n = 0; lam < 4; ++lam)
-#pragma unroll
-            for (int mu = lam; mu < 4; ++mu, ++n) cs[n] = conn(nu * 16 + lam * 4 + mu);
-#pragma unroll
-        for (int lam = 0, n = 0; lam < 4; ++lam)
-#pragma unroll
-            for (int mu = lam; mu < 4; ++mu, ++n) {
-                nd[lam] += T[mu][nu] * cs[n];
-                if (mu != lam) nd[mu] += T[lam][nu] * cs[n];
-            }
-    }
-    dudt[UU] += nd[0];
-    dudt[U1] += nd[1];
-    dudt[U2] += nd[2];
-    dudt[U3] += nd[3];
-}
-template <class G>
-__device__ __forceinline__ void add_geo_source(const G& g, const GeomDev& gd, long q, const double Psub[NV], double gam,
-                                               double dudt[NV]) {
-    add_geo_source_c(g, [&](int n) { return gd.conn[(long)n * gd.np + q]; }, Psub, gam, dudt);
 }
 
 // ----------------------------------------------------------------- flux-CT
@@ -230,552 +66,6 @@ __global__ void __launch_bounds__(BS) ct_rewrite_kernel(BlockDims b, FluxVars<R>
         F3[B2][c] = R(-0.5) * (e1[c] + e1[c + b.s2]);
         F3[B3][c] = R(0);
     }
-}
-
-// Flux divergence of all 8 variables of zone c (FluxDivHelper form:
-// -(sum_d A_d (F_d(hi) - F_d(lo))) / V), with the flux-CT B fluxes
-// evaluated from the EMFs when `ct` is set.
-template <typename R>
-__device__ __forceinline__ void zone_divergence(const BlockDims& b, const FluxVars<const R>& F, const R* __restrict__ emf,
-                                                long c, bool ct, double dudt[NV], bool skip_b = false) {
-    const double A1 = b.dx2 * b.dx3, A2 = b.dx1 * b.dx3, A3 = b.dx1 * b.dx2, V = b.dx1 * b.dx2 * b.dx3;
-    const double iV = 1. / V;   // one division per zone instead of eight
-    const Vars<const R>& F1 = F[0];
-    const Vars<const R>& F2 = F[1];
-    const Vars<const R>& F3 = F[2];
-    const long s2 = b.s2, s3 = b.s3;
-    const int nd = b.ndim;
-    double f1lo[NV], f1hi[NV], f2lo[NV], f2hi[NV], f3lo[NV], f3hi[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        f1lo[v] = f1hi[v] = f2lo[v] = f2hi[v] = f3lo[v] = f3hi[v] = 0.;
-        if (skip_b && v >= B1) continue;   // face-centred B: the cell B comes from the faces
-        f1lo[v] = (double)F1[v][c];
-        f1hi[v] = (double)F1[v][c + 1];
-        if (nd >= 2 && !(ct && v >= B1)) { f2lo[v] = (double)F2[v][c]; f2hi[v] = (double)F2[v][c + s2]; }
-        if (nd == 3 && !(ct && v >= B1)) { f3lo[v] = (double)F3[v][c]; f3hi[v] = (double)F3[v][c + s3]; }
-    }
-    if (ct) {
-        const R* e1 = emf;
-        const R* e2 = emf + b.nc;
-        const R* e3 = emf + 2 * b.nc;
-        f1lo[B1] = 0.; f1hi[B1] = 0.;
-        f1lo[B2] = (double)(R(0.5) * (e3[c] + e3[c + s2]));
-        f1hi[B2] = (double)(R(0.5) * (e3[c + 1] + e3[c + 1 + s2]));
-        f2lo[B1] = (double)(R(-0.5) * (e3[c] + e3[c + 1]));
-        f2hi[B1] = (double)(R(-0.5) * (e3[c + s2] + e3[c + s2 + 1]));
-        f2lo[B2] = 0.; f2hi[B2] = 0.;
-        if (nd == 3) {
-            f1lo[B3] = (double)(R(-0.5) * (e2[c] + e2[c + s3]));
-            f1hi[B3] = (double)(R(-0.5) * (e2[c + 1] + e2[c + 1 + s3]));
-            f2lo[B3] = (double)(R(0.5) * (e1[c] + e1[c + s3]));
-            f2hi[B3] = (double)(R(0.5) * (e1[c + s2] + e1[c + s2 + s3]));
-            f3lo[B1] = (double)(R(0.5) * (e2[c] + e2[c + 1]));
-            f3hi[B1] = (double)(R(0.5) * (e2[c + s3] + e2[c + s3 + 1]));
-            f3lo[B2] = (double)(R(-0.5) * (e1[c] + e1[c + s2]));
-            f3hi[B2] = (double)(R(-0.5) * (e1[c + s3] + e1[c + s3 + s2]));
-            f3lo[B3] = 0.; f3hi[B3] = 0.;
-        } else {
-            // 2D: B3 keeps its Riemann fluxes
-            f2lo[B3] = (double)F2[B3][c];
-            f2hi[B3] = (double)F2[B3][c + s2];
-        }
-    }
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        double du = (A1 * f1hi[v] - A1 * f1lo[v]);
-        if (nd >= 2) du += (A2 * f2hi[v] - A2 * f2lo[v]);
-        if (nd == 3) du += (A3 * f3hi[v] - A3 * f3lo[v]);
-        dudt[v] = -du * iV;
-    }
-}
-
-__device__ __forceinline__ double zone_ndt(const BlockDims& b, double c1, double c2, double c3) {
-    // GRMHD::EstimateTimestep, grmhd.cpp:320-322, with c_d = max(cmax_d, cmin_d)
-    return 1.0 / (1 / (b.dx1 / c1) + 1 / (b.dx2 / c2) + 1 / (b.dx3 / c3));
-}
-
-// Block-wide min / max (wavefront shuffles, then LDS across the block's waves).
-__device__ __forceinline__ double block_min(double v) {
-    __shared__ double red[1024 / 64];
-    v = wave_min(v);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) red[w] = v;
-    __syncthreads();
-    double m = red[0];
-    for (int q = 1; q < (int)(blockDim.x >> 6); ++q) m = fmin(m, red[q]);
-    return m;
-}
-__device__ __forceinline__ double block_max(double v) {
-    __shared__ double red[1024 / 64];
-    v = wave_max(v);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) red[w] = v;
-    __syncthreads();
-    double m = red[0];
-    for (int q = 1; q < (int)(blockDim.x >> 6); ++q) m = fmax(m, red[q]);
-    return m;
-}
-
-// Corner EMFs of flux-CT (b_flux_ct.cpp:331-342) evaluated from the Riemann
-// B fluxes at corner c.
-template <typename R>
-__device__ __forceinline__ R emf3_at(const R* F1B2, const R* F2B1, long c, long s2) {
-    return R(0.25) * (F1B2[c] + F1B2[c - s2] - F2B1[c] - F2B1[c - 1]);
-}
-template <typename R>
-__device__ __forceinline__ R emf1_at(const R* F2B3, const R* F3B2, long c, long s2, long s3) {
-    return R(0.25) * (F2B3[c] + F2B3[c - s3] - F3B2[c] - F3B2[c - s2]);
-}
-template <typename R>
-__device__ __forceinline__ R emf2_at(const R* F3B1, const R* F1B3, long c, long s3) {
-    return R(0.25) * (F3B1[c] + F3B1[c - 1] - F1B3[c] - F1B3[c - s3]);
-}
-
-// Divergence of zone c with the flux-CT B fluxes (b_flux_ct.cpp:347-369) built
-// from EMFs computed here from the Riemann fluxes, so neither the EMFs nor the
-// rewritten B fluxes make a trip through HBM.
-// ND (2 or 3) fixes the dimensionality at compile time; ND = 0 reads b.ndim.
-template <typename R, int ND = 0>
-__device__ __forceinline__ void zone_divergence_ct(const BlockDims& b, const R* __restrict__ F, long c, double dudt[NV]) {
-    const double A1 = b.dx2 * b.dx3, A2 = b.dx1 * b.dx3, A3 = b.dx1 * b.dx2, V = b.dx1 * b.dx2 * b.dx3;
-    const double iV = 1. / V;   // one division per zone instead of eight
-    const R* F1 = F;
-    const R* F2 = F + 8 * b.nc;
-    const R* F3 = F + 16 * b.nc;
-    const long s2 = b.s2, s3 = b.s3, nc = b.nc;
-    const int nd = ND ? ND : b.ndim;
-    double f1lo[NV], f1hi[NV], f2lo[NV], f2hi[NV], f3lo[NV], f3hi[NV];
-#pragma unroll
-    for (int v = 0; v < B1; ++v) {
-        f1lo[v] = (double)F1[v * nc + c];
-        f1hi[v] = (double)F1[v * nc + c + 1];
-        f2lo[v] = (double)F2[v * nc + c];
-        f2hi[v] = (double)F2[v * nc + c + s2];
-        if (nd == 3) { f3lo[v] = (double)F3[v * nc + c]; f3hi[v] = (double)F3[v * nc + c + s3]; }
-        else { f3lo[v] = 0.; f3hi[v] = 0.; }
-    }
-    const R* F1B2 = F1 + B2 * nc;
-    const R* F2B1 = F2 + B1 * nc;
-    const R e3_00 = emf3_at(F1B2, F2B1, c, s2), e3_10 = emf3_at(F1B2, F2B1, c + 1, s2);
-    const R e3_01 = emf3_at(F1B2, F2B1, c + s2, s2), e3_11 = emf3_at(F1B2, F2B1, c + s2 + 1, s2);
-    f1lo[B1] = 0.; f1hi[B1] = 0.;
-    f1lo[B2] = (double)(R(0.5) * (e3_00 + e3_01));
-    f1hi[B2] = (double)(R(0.5) * (e3_10 + e3_11));
-    f2lo[B1] = (double)(R(-0.5) * (e3_00 + e3_10));
-    f2hi[B1] = (double)(R(-0.5) * (e3_01 + e3_11));
-    f2lo[B2] = 0.; f2hi[B2] = 0.;
-    f3lo[B1] = f3hi[B1] = f3lo[B2] = f3hi[B2] = f3lo[B3] = f3hi[B3] = 0.;
-    if (nd == 3) {
-        const R* F2B3 = F2 + B3 * nc;
-        const R* F3B2 = F3 + B2 * nc;
-        const R* F3B1 = F3 + B1 * nc;
-        const R* F1B3 = F1 + B3 * nc;
-        const R e1_000 = emf1_at(F2B3, F3B2, c, s2, s3), e1_010 = emf1_at(F2B3, F3B2, c + s2, s2, s3);
-        const R e1_001 = emf1_at(F2B3, F3B2, c + s3, s2, s3), e1_011 = emf1_at(F2B3, F3B2, c + s2 + s3, s2, s3);
-        const R e2_000 = emf2_at(F3B1, F1B3, c, s3), e2_100 = emf2_at(F3B1, F1B3, c + 1, s3);
-        const R e2_001 = emf2_at(F3B1, F1B3, c + s3, s3), e2_101 = emf2_at(F3B1, F1B3, c + s3 + 1, s3);
-        f1lo[B3] = (double)(R(-0.5) * (e2_000 + e2_001));
-        f1hi[B3] = (double)(R(-0.5) * (e2_100 + e2_101));
-        f2lo[B3] = (double)(R(0.5) * (e1_000 + e1_001));
-        f2hi[B3] = (double)(R(0.5) * (e1_010 + e1_011));
-        f3lo[B1] = (double)(R(0.5) * (e2_000 + e2_100));
-        f3hi[B1] = (double)(R(0.5) * (e2_001 + e2_101));
-        f3lo[B2] = (double)(R(-0.5) * (e1_000 + e1_010));
-        f3hi[B2] = (double)(R(-0.5) * (e1_001 + e1_011));
-    } else {
-        // 2D: B3 keeps its Riemann fluxes
-        f1lo[B3] = (double)F1[B3 * nc + c];
-        f1hi[B3] = (double)F1[B3 * nc + c + 1];
-        f2lo[B3] = (double)F2[B3 * nc + c];
-        f2hi[B3] = (double)F2[B3 * nc + c + s2];
-    }
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        double du = (A1 * f1hi[v] - A1 * f1lo[v]);
-        du += (A2 * f2hi[v] - A2 * f2lo[v]);
-        if (nd == 3) du += (A3 * f3hi[v] - A3 * f3lo[v]);
-        dudt[v] = -du * iV;
-    }
-}
-
-// The U->P solver of inverter/type (inverter.cpp:53-70): INV 0 onedw, 1 Kastaun.
-template <int INV, class G>
-__device__ __forceinline__ int invert_zone(const G& g, const double U[NV], double P[NV], const StepConsts& cst) {
-    if constexpr (INV == 1) return u_to_p_kastaun(g, U, P, cst.gam, cst.floors, cst.iter_max, cst.err_tol);
-    else return u_to_p_onedw(g, U, P, cst.gam, cst.iter_max, cst.err_tol);
-}
-
-// ------------------------------------------------------- fused stage update
-// Stage 1 (gam0 = 0 and U_sub == U_full) reads the state once: 0*U + 1*U == U.
-// BM: 0 no B transport (1-D), 1 flux-CT EMFs from the face fluxes, 2 face-centred
-// B (B_CT): the cell B is the average of the stage's new faces fB (B_CT::BlockUtoP,
-// b_ct.cpp:173-205, which the reference runs before the inversion).
-template <typename R, bool DO_DT, int BM, int GEO, int INV = 0, bool PK = false>
-__global__ void __launch_bounds__(BS, UpdateOcc<GEO>::min_blocks)
-update_kernel(BlockDims b, StepConsts cst, GeomDev gd, int stage, const R* __restrict__ F, const R* __restrict__ ctop,
-              const double* __restrict__ Usub, const double* Ufull, const double* __restrict__ Psub,
-              double* Uout, double* __restrict__ Pout, float* __restrict__ Pout32,
-              int* __restrict__ pflag, int* __restrict__ fflag, int* __restrict__ fail_list,
-              DeviceState* __restrict__ ds, double* __restrict__ dt_part, const double* __restrict__ fB,
-              const BlockEntry* __restrict__ pk) {
-    if constexpr (PK) {
-        const long blk = pack_select(pk, b, gd);
-        const long sv = blk * NV * b.nc;
-        F = pack_at(F, 3 * sv);
-        ctop = pack_at(ctop, blk * 3 * b.nc);
-        Usub = pack_at(Usub, sv); Ufull = pack_at(Ufull, sv); Psub = pack_at(Psub, sv);
-        Uout = pack_at(Uout, sv); Pout = pack_at(Pout, sv); Pout32 = pack_at(Pout32, sv);
-        pflag = pack_at(pflag, blk * b.nc); fflag = pack_at(fflag, blk * b.nc); fail_list = pack_at(fail_list, blk * b.nc);
-        ds += blk;
-        dt_part = pack_at(dt_part, blk * gridDim.x);
-    }
-    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = t < (unsigned)ninterior(b);
-    double ndt = DBL_MAX;
-    if (active) {
-        int k, j, i;
-        interior_index(b, t, k, j, i);
-        const long c = (long)k * b.s3 + (long)j * b.s2 + i;
-        const double gam = cst.gam;
-        double dudt[NV];
-        if (BM == 1) zone_divergence_ct<R>(b, F, c, dudt);
-        else zone_divergence<R>(b, flux_vars_of(F, b.nc), nullptr, c, false, dudt, BM == 2);
-        if constexpr (GEO) {
-            double Ps[NV];
-#pragma unroll
-            for (int v = 0; v < NV; ++v) Ps[v] = Psub[v * b.nc + c];
-            const long q = (long)j * gd.gn1 + i;
-            CachedGeom<double> g(gd.g[GLOC_CENTER], gd.np, q);
-            add_geo_source(g, gd, q, Ps, gam, dudt);
-        }
-        const double g0 = cst.gam0[stage - 1], g1 = cst.gam1[stage - 1];
-        const double beta_dt = cst.beta[stage - 1] * ds->dt;
-        const bool same = (g0 == 0.) && (Usub == Ufull);
-        double U[NV], P[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const double uf = Ufull[v * b.nc + c];
-            const double u = same ? uf : g0 * Usub[v * b.nc + c] + g1 * uf;
-            U[v] = 1.0 * u + beta_dt * dudt[v];
-        }
-        if constexpr (BM == 2) {
-            const long f = (long)k * b.fs3 + (long)j * b.fs2 + i;
-            U[B1] = (fB[f] + fB[f + 1]) / 2;
-            U[B2] = (fB[b.nf + f] + fB[b.nf + f + b.fs2]) / 2;
-            U[B3] = (b.ndim > 2) ? (fB[2 * b.nf + f] + fB[2 * b.nf + f + b.fs3]) / 2 : fB[2 * b.nf + f];
-        }
-        // U->P guess: the stage's starting primitives (kharma_driver.cpp:379-384)
-#pragma unroll
-        for (int v = 0; v < 5; ++v) P[v] = Psub[v * b.nc + c];
-        int pf = 0, ff = 0;
-        double rf, uf;
-        geom_floors<GEO>(cst, gd, j, i, rf, uf);
-        with_center_geom<GEO>(gd, j, i, [&](const auto& g) {
-            pf = invert_zone<INV>(g, U, P, cst);
-            const int ff0 = (pf / F_GEOM_RHO) * F_GEOM_RHO;
-            pf = pf % F_GEOM_RHO;
-            const double gd_ = g.gdet();
-            const double igd = rcp(gd_);
-            P[B1] = U[B1] * igd; P[B2] = U[B2] * igd; P[B3] = U[B3] * igd;
-            FourVec<double> D;
-            calc_4vecs<double>(g, P, D);
-            ff = ff0;
-            if (cst.floors.on) ff = floors_zone(g, P, U, D, gam, cst.floors, rf, uf, ff0, pf);
-            p_to_u_D(g, P, D, gam, U);
-        });
-        ImageSet s;
-        image_set(b, k, j, i, s);
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            store_with_images(b, s, Uout + v * b.nc, c, U[v], NV * b.nc);
-            store_with_images(b, s, Pout + v * b.nc, c, P[v], NV * b.nc);
-            if (Pout32) store_with_images(b, s, Pout32 + v * b.nc, c, (float)P[v], NV * b.nc);
-        }
-        store_with_images(b, s, pflag, c, pf, b.nc);
-        fflag[c] = ff;
-        if (pf > 0) {
-            const int slot = atomicAdd(&ds->fail_count[stage - 1], 1);
-            fail_list[slot] = (int)c;
-        }
-        if (DO_DT) {
-            const double n = zone_ndt(b, (double)ctop[c], b.ndim > 1 ? (double)ctop[b.nc + c] : 0.,
-                                      b.ndim > 2 ? (double)ctop[2 * b.nc + c] : 0.);
-            if (!(n != n)) ndt = n;
-        }
-    }
-    if (DO_DT) {
-        const double m = block_min(ndt);
-        if (threadIdx.x == 0) dt_part[blockIdx.x] = m;
-    }
-}
-
-// ------------------------------------------- curved-space stage update, split
-// In Kerr-Schild geometry the fused update needs ~240 VGPRs (two waves per
-// SIMD) and spends most of its time waiting.  It runs as two kernels instead:
-// combine_kernel (flux divergence, geometric source, RK combination -> U) and
-// recover_kernel (U->P, floors, P->U, flags).  The arithmetic is the same as
-// the fused kernel's, so the results are bit-identical; the cost is one extra
-// write and read of U (128 bytes per zone).
-//
-// Both walk the interior in (j, k, i) order, i fastest, with the workgroups
-// renumbered so each XCD (workgroup w runs on XCD w % 8) owns one contiguous
-// range of j: the axisymmetric geometry tables ([comp][j][i]) a workgroup
-// reads then stay within one eighth of the table per XCD L2.
-// Waves per SIMD the two halves are built for (the second launch bound).  The
-// staged 3-D recovery on 64-wide tiles runs 4 (128 VGPRs with a 12-byte spill
-// instead of 140: 262 -> 234 us on the 192x128x128 torus); on 32-wide tiles
-// (28-byte spill) 4 waves measured 1 % slower, and the recovery in the
-// normal-observer frame (182-241 VGPRs) and the unstaged ones would spill
-// hundreds of bytes, so those keep their natural allocation.  The combine keeps
-// its 2 waves: a 3-wave bound (168 VGPRs, 20-90 byte spill) measured 1-7 % slower.
-template <int FRAME, bool STG, int TI> struct RecOcc {
-    static constexpr int w = (STG && FRAME != 1 && TI == 64) ? 4 : 1;
-};
-constexpr unsigned N_XCD = 8;
-__device__ __forceinline__ unsigned xcd_logical_block(unsigned b, unsigned nb) {
-    const unsigned x = b % N_XCD, r = b / N_XCD, q = nb / N_XCD, m = nb % N_XCD;
-    return x * q + (x < m ? x : m) + r;
-}
-__device__ __forceinline__ void interior_index_jki(const BlockDims& b, unsigned t, int& k, int& j, int& i) {
-    const unsigned n3 = (unsigned)(b.ndim > 2 ? b.nx3 : 1);
-    const unsigned row = t / (unsigned)b.nx1;
-    const unsigned jj = row / n3;
-    i = b.is + (int)(t - row * (unsigned)b.nx1);
-    k = b.ks + (int)(row - jj * n3);
-    j = b.js + (int)jj;
-}
-
-// In 3-D the recover kernel runs on tiles of TI = 64 x1 cells by 4 x3 rows at
-// one x2 row, one x3 row per wavefront: the four wavefronts of a work-group
-// share the geometry of their 64 (j, i) columns (the 22 metric components and
-// the 2 geometric floors), which the work-group stages once in LDS as
-// [component][64] instead of each zone loading its own.  A block whose x1 width
-// is an odd multiple of 32 (the 96-wide blocks of a 2x2x4 mesh of the
-// 192x128x128 torus) runs TI = 32 by 8 rows instead, two rows per wavefront, so
-// that no tile is half empty.  Tiles are numbered i fastest, then k, then j, and
-// renumbered per XCD as above.  Each zone's U and P loads are issued before the
-// staging so that they overlap it (272 -> 262 us on the 192x128x128 torus).
-// (Staging the connection as well and adding the geometric source here instead
-// of in the combine shortens the combine -- 75-102 VGPRs instead of 190-254 --
-// but slows the recovery by more: measured 223 + 469 against 371 + 262 us for
-// the split stage-2 update.)
-constexpr int STG_RECOVER = GEO_NCOMP + 2;
-template <int TI> __host__ __device__ __forceinline__ int tiles_i(const BlockDims& b) { return (b.nx1 + TI - 1) / TI; }
-template <int TI> __host__ __device__ __forceinline__ int tiles_k(const BlockDims& b) {
-    return (b.nx3 + BS / TI - 1) / (BS / TI);
-}
-// The recovery's tile width for block b: 32 where it leaves fewer idle lanes.
-static inline int recover_tile_i(const BlockDims& b) {
-    return (tiles_i<32>(b) * 32 - b.nx1 < tiles_i<64>(b) * 64 - b.nx1) ? 32 : 64;
-}
-static inline long update_tiles_host(const BlockDims& b) {
-    return recover_tile_i(b) == 32 ? (long)tiles_i<32>(b) * tiles_k<32>(b) * b.nx2
-                                   : (long)tiles_i<64>(b) * tiles_k<64>(b) * b.nx2;
-}
-// Zone (k, j, i) of this thread; i0 is the tile's first x1 cell.
-template <int TI>
-__device__ __forceinline__ bool tile_zone(const BlockDims& b, int& k, int& j, int& i, int& i0) {
-    const unsigned lb = xcd_logical_block(blockIdx.x, gridDim.x);
-    const unsigned nti = (unsigned)tiles_i<TI>(b), ntk = (unsigned)tiles_k<TI>(b);
-    const unsigned ti = lb % nti, rest = lb / nti;
-    const unsigned tk = rest % ntk, jj = rest / ntk;
-    const int row = (TI == 64) ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / TI)) : (int)(threadIdx.x / TI);
-    i0 = b.is + (int)ti * TI;
-    i = i0 + (int)(threadIdx.x % TI);
-    k = b.ks + (int)tk * (BS / TI) + row;
-    j = b.js + (int)jj;
-    return i <= b.ie && k <= b.ke;
-}
-// Stage the tile's metric and floors (x1 clamped to the table for a ragged
-// last tile) into sg; every thread of the work-group calls it.
-template <int TI>
-__device__ __forceinline__ void stage_recover_geometry(const GeomDev& gd, int j, int i0, double* sg) {
-    const int lane = (int)(threadIdx.x % TI);
-    const int w = (TI == 64) ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x / TI)) : (int)(threadIdx.x / TI);
-    const long q = (long)j * gd.gn1 + min(i0 + lane, gd.gn1 - 1);
-#pragma unroll
-    for (int c0 = 0; c0 < STG_RECOVER; c0 += BS / TI) {
-        const int comp = c0 + w;
-        if (comp < STG_RECOVER)
-            sg[comp * TI + lane] = comp < GEO_NCOMP ? gd.g[GLOC_CENTER][(long)comp * gd.np + q]
-                                                    : gd.flr[(long)(comp - GEO_NCOMP) * gd.np + q];
-    }
-    __syncthreads();
-}
-
-// ND: dimensionality (flux-CT for 2 and 3); SAME: stage with gam0 = 0 and
-// U_sub == U_full, which reads the state once (0*U + 1*U == U).
-template <typename R, bool DO_DT, int ND, bool SAME, bool PK>
-__global__ void __launch_bounds__(BS)
-combine_kernel(BlockDims b, StepConsts cst, GeomDev gd, int stage, const R* __restrict__ F, const R* __restrict__ ctop,
-               const double* __restrict__ Usub, const double* Ufull, const double* __restrict__ Psub, double* Uout,
-               const DeviceState* __restrict__ ds, double* __restrict__ dt_part, const BlockEntry* __restrict__ pk) {
-    if constexpr (PK) {
-        const long blk = pack_select(pk, b, gd);
-        const long sv = blk * NV * b.nc;
-        F = pack_at(F, 3 * sv);
-        ctop = pack_at(ctop, blk * 3 * b.nc);
-        Usub = pack_at(Usub, sv); Ufull = pack_at(Ufull, sv); Psub = pack_at(Psub, sv); Uout = pack_at(Uout, sv);
-        ds += blk;
-        dt_part = pack_at(dt_part, blk * gridDim.x);
-    }
-    const unsigned t = xcd_logical_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    const bool active = t < (unsigned)ninterior(b);
-    double ndt = DBL_MAX;
-    if (active) {
-        int k, j, i;
-        interior_index_jki(b, t, k, j, i);
-        const long c = (long)k * b.s3 + (long)j * b.s2 + i;
-        const double g0 = cst.gam0[stage - 1], g1 = cst.gam1[stage - 1];
-        // The geometric source (flux.cpp:395-444) of the stage's primitives.  The
-        // FP32-flux form computes it first, before the state and the fluxes are
-        // loaded (100 instead of 174-190 VGPRs, 1-2 % faster); the FP64 form keeps
-        // it after the divergence (first measured 2 % slower there).  Both add
-        // it to the divergence in the same order, so the results are the same.
-        constexpr bool SRC_FIRST = sizeof(R) == 4;
-        auto source = [&](double acc[NV]) {
-            double Ps[NV];
-#pragma unroll
-            for (int v = 0; v < NV; ++v) Ps[v] = Psub[v * b.nc + c];
-            const long q = (long)j * gd.gn1 + i;
-            CachedGeom<double> g(gd.g[GLOC_CENTER], gd.np, q);
-            add_geo_source(g, gd, q, Ps, cst.gam, acc);
-        };
-        double dS[NV] = {0., 0., 0., 0., 0., 0., 0., 0.};
-        if constexpr (SRC_FIRST) source(dS);
-        double Ub[NV];   // the stage's base state, loaded early so its latency overlaps the rest
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-            const double uf = Ufull[v * b.nc + c];
-            Ub[v] = SAME ? uf : g0 * Usub[v * b.nc + c] + g1 * uf;
-        }
-        double dudt[NV];
-        if constexpr (ND > 1) zone_divergence_ct<R, ND>(b, F, c, dudt);
-        else zone_divergence<R>(b, flux_vars_of(F, b.nc), nullptr, c, false, dudt);
-        if constexpr (SRC_FIRST) {
-#pragma unroll
-            for (int v = UU; v <= U3; ++v) dudt[v] += dS[v];
-        } else {
-            source(dudt);
-        }
-        const double beta_dt = cst.beta[stage - 1] * ds->dt;
-#pragma unroll
-        for (int v = 0; v < NV; ++v) Uout[v * b.nc + c] = 1.0 * Ub[v] + beta_dt * dudt[v];
-        if (DO_DT) {
-            const double n = zone_ndt(b, (double)ctop[c], ND > 1 ? (double)ctop[b.nc + c] : 0.,
-                                      ND > 2 ? (double)ctop[2 * b.nc + c] : 0.);
-            if (!(n != n)) ndt = n;
-        }
-    }
-    if (DO_DT) {
-        const double m = block_min(ndt);
-        if (threadIdx.x == 0) dt_part[blockIdx.x] = m;
-    }
-}
-
-// U->P with the stage's starting primitives as guess (kharma_driver.cpp:379-384),
-// B from U, floors in frame FRAME, P->U; U is read from and written back to Uout.
-// One zone (k, j, i) at c, whose U and guess P the caller has loaded.
-template <int FRAME, int INV, bool STG, int TI>
-__device__ __forceinline__ void recover_zone(const BlockDims& b, const StepConsts& cst, const GeomDev& gd, int stage,
-                                             double* Uout, double* __restrict__ Pout,
-                                             float* __restrict__ Pout32, int* __restrict__ pflag,
-                                             int* __restrict__ fflag, int* __restrict__ fail_list,
-                                             DeviceState* __restrict__ ds, double* __restrict__ Ustar,
-                                             const double* sg, int k, int j, int i, long c, double (&U)[NV],
-                                             double (&P)[NV]) {
-    const double gam = cst.gam;
-    int pf = 0, ff = 0;
-    double rf, uf;
-    const int lane = (int)(threadIdx.x % TI);
-    if (Ustar) {   // the stage's U* for the differentiation form's record
-#pragma unroll
-        for (int v = 0; v < NV; ++v) Ustar[v * b.nc + c] = U[v];
-    }
-    if constexpr (STG) {
-        rf = sg[GEO_NCOMP * TI + lane];
-        uf = sg[(GEO_NCOMP + 1) * TI + lane];
-    } else {
-        geom_floors<1>(cst, gd, j, i, rf, uf);
-    }
-    {
-        CachedGeom<double> g(STG ? sg : gd.g[GLOC_CENTER], STG ? TI : gd.np, STG ? lane : (long)j * gd.gn1 + i);
-        pf = invert_zone<INV>(g, U, P, cst);
-        const int ff0 = (pf / F_GEOM_RHO) * F_GEOM_RHO;
-        pf = pf % F_GEOM_RHO;
-        const double gd_ = g.gdet();
-        const double igd = rcp(gd_);
-        P[B1] = U[B1] * igd; P[B2] = U[B2] * igd; P[B3] = U[B3] * igd;
-        FourVec<double> D;
-        calc_4vecs<double, true>(g, P, D);
-        ff = ff0;
-        if (cst.floors.on) ff = floors_zone<FRAME>(g, P, U, D, gam, cst.floors, rf, uf, ff0, pf);
-        p_to_u_D(g, P, D, gam, U);
-    }
-    ImageSet s;
-    image_set(b, k, j, i, s);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        store_with_images(b, s, Uout + v * b.nc, c, U[v], NV * b.nc);
-        store_with_images(b, s, Pout + v * b.nc, c, P[v], NV * b.nc);
-        if (Pout32) store_with_images(b, s, Pout32 + v * b.nc, c, (float)P[v], NV * b.nc);
-    }
-    store_with_images(b, s, pflag, c, pf, b.nc);
-    fflag[c] = ff;
-    if (pf > 0) {
-        const int slot = atomicAdd(&ds->fail_count[stage - 1], 1);
-        fail_list[slot] = (int)c;
-    }
-}
-
-template <int FRAME, int INV, bool STG, bool PK, int TI = 64>
-__global__ void __launch_bounds__(BS, (RecOcc<FRAME, STG, TI>::w))
-recover_kernel(BlockDims b, StepConsts cst, GeomDev gd, int stage, const double* __restrict__ Psub, double* Uout,
-               double* __restrict__ Pout, float* __restrict__ Pout32, int* __restrict__ pflag,
-               int* __restrict__ fflag, int* __restrict__ fail_list, DeviceState* __restrict__ ds,
-               double* __restrict__ Ustar, const BlockEntry* __restrict__ pk) {
-    __shared__ double sg[STG ? STG_RECOVER * TI : 1];
-    if constexpr (PK) {
-        const long blk = pack_select(pk, b, gd);
-        const long sv = blk * NV * b.nc;
-        Psub = pack_at(Psub, sv); Uout = pack_at(Uout, sv); Pout = pack_at(Pout, sv); Pout32 = pack_at(Pout32, sv);
-        Ustar = pack_at(Ustar, sv);
-        pflag = pack_at(pflag, blk * b.nc); fflag = pack_at(fflag, blk * b.nc); fail_list = pack_at(fail_list, blk * b.nc);
-        ds += blk;
-    }
-    constexpr int NP = 5;   // the guess: the fluid primitives (B follows from U)
-    int k, j, i;
-    long c;
-    double U[NV], P[NV];
-    if constexpr (STG) {
-        // the zone's U and P are requested before the tile's geometry is staged,
-        // so that their latency overlaps the staging and its barrier
-        int i0;
-        const bool active = tile_zone<TI>(b, k, j, i, i0);
-        c = (long)k * b.s3 + (long)j * b.s2 + i;
-        if (active) {
-#pragma unroll
-            for (int v = 0; v < NV; ++v) U[v] = Uout[v * b.nc + c];
-#pragma unroll
-            for (int v = 0; v < NP; ++v) P[v] = Psub[v * b.nc + c];
-        }
-        stage_recover_geometry<TI>(gd, j, i0, sg);
-        if (!active) return;
-    } else {
-        const unsigned t = xcd_logical_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-        if (t >= (unsigned)ninterior(b)) return;
-        interior_index_jki(b, t, k, j, i);
-        c = (long)k * b.s3 + (long)j * b.s2 + i;
-#pragma unroll
-        for (int v = 0; v < NV; ++v) U[v] = Uout[v * b.nc + c];
-#pragma unroll
-        for (int v = 0; v < NP; ++v) P[v] = Psub[v * b.nc + c];
-    }
-    recover_zone<FRAME, INV, STG, TI>(b, cst, gd, stage, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, Ustar, sg, k, j,
-                                  i, c, U, P);
 }
 
 // Inverter::FixUtoP (inverter/fixup.cpp:47-156) on the zones listed by the
@@ -1484,8 +774,8 @@ hipError_t launch_flux_divergence(const BlockDims& b, int prec, const FluxVars<v
 // DetermineGRMHDFloors.  A zone is marked when the inverter's floor bits or the
 // floors' flags are set, or when `fixed` marks it (within the horizon buffer,
 // polar rows).  Interior zones only.
-// STG (3-D curved space): the zones run on the recovery's tiles, with the tile's
-// metric and floors staged in LDS once, as the recovery does: 132 instead of 188
+// STG (3-D curved space): the zones run on the stage update's tiles, with the tile's
+// metric and floors staged in LDS once, as the update does: 132 instead of 188
 // VGPRs (3 waves per SIMD instead of 2) and 344 -> 319 us per launch on the FP64
 // 192x128x128 torus, with the same marks.  (A 4-wave bound spills 36 B per lane and
 // measured the same.)
@@ -1495,7 +785,7 @@ fofc_mark_kernel(BlockDims b, StepConsts cst, GeomDev gd, int stage, const doubl
                  const double* __restrict__ Usub, const double* Ufull, const double* __restrict__ Psub,
                  const int* __restrict__ fixed, const DeviceState* __restrict__ ds, int* __restrict__ mark,
                  bool images) {
-    __shared__ double sg[STG ? STG_RECOVER * TI : 1];
+    __shared__ double sg[STG ? STG_GEOM * TI : 1];
     int k, j, i, i0 = 0;
     bool active;
     if constexpr (STG) {
@@ -1524,7 +814,7 @@ fofc_mark_kernel(BlockDims b, StepConsts cst, GeomDev gd, int stage, const doubl
         for (int v = 0; v < 5; ++v) P[v] = Psub[v * b.nc + c];
     }
     if constexpr (STG) {
-        stage_recover_geometry<TI>(gd, j, i0, sg);
+        stage_tile_geometry<TI>(gd, j, i0, sg);
         if (!active) return;
     }
     double rf, uf;
@@ -1573,7 +863,7 @@ hipError_t launch_fofc_mark(const BlockDims& b, const StepConsts& c, const GeomD
                        fixed, ds, mark, images)
     if (b.geo && b.ndim == 3) {
         const dim3 gt((unsigned)update_tiles_host(b));
-        const bool ti32 = recover_tile_i(b) == 32;
+        const bool ti32 = tile_width(b) == 32;
         if (c.inverter == 1) { if (ti32) KH_MARK(1, 1, true, 32, gt); else KH_MARK(1, 1, true, 64, gt); }
         else { if (ti32) KH_MARK(1, 0, true, 32, gt); else KH_MARK(1, 0, true, 64, gt); }
     } else if (b.geo) {
@@ -1585,141 +875,6 @@ hipError_t launch_fofc_mark(const BlockDims& b, const StepConsts& c, const GeomD
     return hipGetLastError();
 }
 
-template <typename R, bool PK>
-static void launch_update_geo_k(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int stage, bool do_dt,
-                              const void* F, const void* ctop, const double* Usub, const double* Ufull,
-                              const double* Psub, double* Uout, double* Pout, float* Pout32, int* pflag, int* fflag,
-                              int* fail_list, DeviceState* ds, double* dt_part, hipStream_t s, int parts,
-                              double* Ustar, const Pack* pk) {
-    const dim3 g = pack_grid(grid_for(ninterior_host(b)), pk);
-    const bool rstg = b.ndim == 3;   // recover on LDS-staged tiles
-    const bool ti32 = recover_tile_i(b) == 32;
-    const dim3 gr = rstg ? pack_grid(dim3((unsigned)update_tiles_host(b)), pk) : g;
-    const BlockEntry* pd = pack_dev(pk);
-    const bool same = (c.gam0[stage - 1] == 0.) && (Usub == Ufull);
-    if (parts & 1) {
-#define KH_CMB(DT, ND, SAME)                                                                                          \
-    hipLaunchKernelGGL((combine_kernel<R, DT, ND, SAME, PK>), g, dim3(BS), 0, s, b, c, gd, stage, (const R*)F, (const R*)ctop, \
-                       Usub, Ufull, Psub, Uout, ds, dt_part, pd)
-#define KH_CMB_ND(DT, SAME) \
-    { if (b.ndim == 3) KH_CMB(DT, 3, SAME); else if (b.ndim == 2) KH_CMB(DT, 2, SAME); else KH_CMB(DT, 1, SAME); }
-    if (do_dt) { if (same) KH_CMB_ND(true, true) else KH_CMB_ND(true, false) }
-    else { if (same) KH_CMB_ND(false, true) else KH_CMB_ND(false, false) }
-#undef KH_CMB_ND
-#undef KH_CMB
-    }
-    if (!(parts & 2)) return;
-#define KH_REC(FR, INV)                                                                                             \
-    do {                                                                                                            \
-        if (rstg && ti32) hipLaunchKernelGGL((recover_kernel<FR, INV, true, PK, 32>), gr, dim3(BS), 0, s, b, c, gd,     \
-                                             stage, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, Ustar, pd);  \
-        else if (rstg) hipLaunchKernelGGL((recover_kernel<FR, INV, true, PK>), gr, dim3(BS), 0, s, b, c, gd, stage, Psub,   \
-                                          Uout, Pout, Pout32, pflag, fflag, fail_list, ds, Ustar, pd);                  \
-        else hipLaunchKernelGGL((recover_kernel<FR, INV, false, PK>), gr, dim3(BS), 0, s, b, c, gd, stage, Psub, Uout, Pout, \
-                                Pout32, pflag, fflag, fail_list, ds, Ustar, pd);                                        \
-    } while (0)
-    if (c.inverter == 1) {
-        if (c.floors.frame == 0) KH_REC(0, 1);
-        else if (c.floors.frame == 1) KH_REC(1, 1);
-        else KH_REC(2, 1);
-    } else {
-        if (c.floors.frame == 0) KH_REC(0, 0);
-        else if (c.floors.frame == 1) KH_REC(1, 0);
-        else KH_REC(2, 0);
-    }
-#undef KH_REC
-}
-template <typename R>
-static void launch_update_geo(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int stage, bool do_dt,
-                              const void* F, const void* ctop, const double* Usub, const double* Ufull,
-                              const double* Psub, double* Uout, double* Pout, float* Pout32, int* pflag, int* fflag,
-                              int* fail_list, DeviceState* ds, double* dt_part, hipStream_t s, int parts = 3,
-                              double* Ustar = nullptr, const Pack* pk = nullptr) {
-    if (pk) launch_update_geo_k<R, true>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag,
-                                         fflag, fail_list, ds, dt_part, s, parts, Ustar, pk);
-    else launch_update_geo_k<R, false>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag,
-                                       fflag, fail_list, ds, dt_part, s, parts, Ustar, pk);
-}
-template <typename R, int GEO, bool PK>
-static void launch_update_t_k(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int stage, bool do_dt,
-                            const void* F, const void* ctop, const double* Usub, const double* Ufull, const double* Psub,
-                            double* Uout, double* Pout, float* Pout32, int* pflag, int* fflag,
-                            int* fail_list, DeviceState* ds, double* dt_part, hipStream_t s, const double* fB,
-                            const Pack* pk) {
-    const dim3 g = pack_grid(grid_for(ninterior_host(b)), pk);
-    const int bm = fB ? 2 : (b.ndim > 1 ? 1 : 0);
-    const BlockEntry* pd = pack_dev(pk);
-#define KH_UPD(DT, BM, INV)                                                                                         \
-    hipLaunchKernelGGL((update_kernel<R, DT, BM, GEO, INV, PK>), g, dim3(BS), 0, s, b, c, gd, stage, (const R*)F, (const R*)ctop, \
-                       Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, fB, pd)
-#define KH_UPD_BM(DT, INV) \
-    { if (bm == 2) KH_UPD(DT, 2, INV); else if (bm == 1) KH_UPD(DT, 1, INV); else KH_UPD(DT, 0, INV); }
-    if (c.inverter == 1) {
-        if (do_dt) KH_UPD_BM(true, 1) else KH_UPD_BM(false, 1)
-    } else {
-        if (do_dt) KH_UPD_BM(true, 0) else KH_UPD_BM(false, 0)
-    }
-#undef KH_UPD_BM
-#undef KH_UPD
-}
-template <typename R, int GEO>
-static void launch_update_t(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int stage, bool do_dt,
-                            const void* F, const void* ctop, const double* Usub, const double* Ufull, const double* Psub,
-                            double* Uout, double* Pout, float* Pout32, int* pflag, int* fflag,
-                            int* fail_list, DeviceState* ds, double* dt_part, hipStream_t s, const double* fB = nullptr,
-                            const Pack* pk = nullptr) {
-    if (pk) launch_update_t_k<R, GEO, true>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32,
-                                            pflag, fflag, fail_list, ds, dt_part, s, fB, pk);
-    else launch_update_t_k<R, GEO, false>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32,
-                                          pflag, fflag, fail_list, ds, dt_part, s, fB, pk);
-}
-hipError_t launch_update_faces(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int prec, int stage,
-                               bool do_dt, const void* F, const void* ctop, const double* Usub, const double* Ufull,
-                               const double* Psub, double* Uout, double* Pout, float* Pout32, int* pflag, int* fflag,
-                               int* fail_list, DeviceState* ds, double* dt_part, const double* fB, hipStream_t s) {
-    if (b.geo || !fB) return hipErrorInvalidValue;
-    if (prec == PREC_SPLIT)
-        launch_update_t<float, 0>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag,
-                                  fail_list, ds, dt_part, s, fB);
-    else
-        launch_update_t<double, 0>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag,
-                                   fail_list, ds, dt_part, s, fB);
-    return hipGetLastError();
-}
-hipError_t launch_update(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int prec, int stage, bool do_dt,
-                         const void* F, const void* ctop, const double* Usub, const double* Ufull, const double* Psub,
-                         double* Uout, double* Pout, float* Pout32, int* pflag, int* fflag,
-                         int* fail_list, DeviceState* ds, double* dt_part, hipStream_t s, const Pack* pk) {
-    if (prec == PREC_SPLIT) {
-        if (b.geo) launch_update_geo<float>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, 3, nullptr, pk);
-        else launch_update_t<float, 0>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, nullptr, pk);
-    } else {
-        if (b.geo) launch_update_geo<double>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, 3, nullptr, pk);
-        else launch_update_t<double, 0>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, nullptr, pk);
-    }
-    return hipGetLastError();
-}
-hipError_t launch_update_parts(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int stage, int parts,
-                               const double* F, const double* Usub, const double* Ufull, const double* Psub, double* Uout,
-                               double* Pout, int* pflag, int* fflag, int* fail_list, DeviceState* ds, hipStream_t s,
-                               double* Ustar) {
-    if (!b.geo) return hipErrorInvalidValue;
-    launch_update_geo<double>(b, c, gd, stage, false, F, nullptr, Usub, Ufull, Psub, Uout, Pout, nullptr, pflag, fflag,
-                              fail_list, ds, nullptr, s, parts, Ustar);
-    return hipGetLastError();
-}
-hipError_t launch_update_recorded(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int stage, bool do_dt,
-                                  const void* F, const void* ctop, const double* Usub, const double* Ufull,
-                                  const double* Psub, double* Uout, double* Pout, int* pflag, int* fflag,
-                                  int* fail_list, DeviceState* ds, double* dt_part, double* Ustar, hipStream_t s) {
-    if (!b.geo)
-        return launch_update(b, c, gd, PREC_FP64, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, nullptr, pflag,
-                             fflag, fail_list, ds, dt_part, s);
-    launch_update_geo<double>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, nullptr, pflag, fflag,
-                              fail_list, ds, dt_part, s, 3, Ustar);
-    return hipGetLastError();
-}
-long update_blocks(const BlockDims& b) { return (ninterior_host(b) + BS - 1) / BS; }
 long divb_blocks(const BlockDims& b) {
     return ((long)(b.nx1 + 1) * (b.nx2 + 1) * ((b.ndim > 2) ? b.nx3 + 1 : 1) + BS - 1) / BS;
 }

@@ -1,0 +1,11 @@
+// kh_update_f32.hip -- the curved-space stage update with FP32 fluxes.
+#include "kh_update_geo.hpp"
+
+namespace kh {
+
+template void launch_update_geo<float>(
+    const BlockDims&, const StepConsts&, const GeomDev&, int, bool, const void*, const void*, const double*,
+    const double*, const double*, double*, double*, float*, int*, int*, int*, DeviceState*, double*, hipStream_t,
+    double*, const Pack*);
+
+}  // namespace kh
