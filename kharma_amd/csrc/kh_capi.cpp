@@ -993,7 +993,9 @@ int kh::driver_stage(kh_driver* d, int stage) {
     double* Uout = (stage == 1) ? d->U1 : d->U0;
     // signal speeds only feed the timestep estimate of the last stage
     const int speeds = (stage == 2) ? SPEEDS_CTOP : SPEEDS_NONE;
-    for (int dir = 1; dir <= bd.ndim; ++dir)
+    if (!d->timing)
+        KH_HIP(launch_flux_stage_all(bd, c, b->geo, b->p.recon, prec, speeds, Psub, Psubf, F, ct, s));
+    else for (int dir = 1; dir <= bd.ndim; ++dir)   // timed by direction
         KH_TIMED(dir - 1, launch_flux_stage(bd, c, b->geo, dir, b->p.recon, prec, speeds, Psub, Psubf,
                                             F + fe * (dir - 1) * NV * bd.nc, ct + fe * (dir - 1) * bd.nc, s));
     if (b->p.fofc) {

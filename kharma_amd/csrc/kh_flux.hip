@@ -128,24 +128,14 @@ __device__ __forceinline__ void face_flux(const StepConsts& c, const BlockDims& 
 // lane and is slower.
 template <typename R, int SPEEDS, bool PK> struct X1Occ { static constexpr int w = sizeof(R) == 4 ? 6 : 1; };
 template <typename R> struct XtOcc { static constexpr int w = sizeof(R) == 4 ? 6 : 1; };
-template <int RECON, int SPEEDS, typename R, typename PT, int GEO, bool PK>
-__global__ void __launch_bounds__(256, (X1Occ<R, SPEEDS, PK>::w))
-flux_x1_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> F,
-               R* __restrict__ cmax_out, R* __restrict__ cmin_out, int j0, int nj, int k0, int nk,
-               const BlockEntry* __restrict__ pk) {
-    __shared__ R sr[NV][256];
-    if constexpr (PK) {
-        const long blk = pack_select(pk, b, gd);
-        P = pack_at(P, blk * NV * b.nc);
-        F = pack_at(F, blk * 3 * NV * b.nc);
-        cmax_out = pack_at(cmax_out, blk * 3 * b.nc);
-        cmin_out = pack_at(cmin_out, blk * 3 * b.nc);
-    }
+template <int RECON, int SPEEDS, typename R, typename PT, int GEO>
+__device__ __forceinline__ void x1_tile(const BlockDims& b, const StepConsts& c, const GeomDev& gd, const Vars<const PT>& P,
+                                        const Vars<R>& F, R* __restrict__ cmax_out, R* __restrict__ cmin_out, int j0,
+                                        int nj, int k0, int nk, unsigned bx, int tid, R (*sr)[256]) {
     const int L = b.nx1 + 2;
-    const int tid = threadIdx.x;
     // cell counts stay below 2^31 (the C ABI bounds a block's size), so the
     // flattened index is divided in 32 bits
-    const unsigned g = blockIdx.x * 255u + (unsigned)tid;
+    const unsigned g = bx * 255u + (unsigned)tid;
     const bool valid = g < (unsigned)L * (unsigned)nj * (unsigned)nk;
     int ii = 0, jf = 0;
     long ci = 0;
@@ -178,20 +168,12 @@ flux_x1_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> 
     for (int v = 0; v < NV; ++v) Pl[v] = sr[v][tid - 1];
     face_flux<1, SPEEDS, R, GEO>(c, b, gd, jf, b.is - 1 + ii, Pl, lo, ci, F, cmax_out, cmin_out);
 }
-
-// X2 / X3 faces.  Transverse columns: flattened (outer, i) with i in [is-1, ie+1]
-// fastest; outer = k (X2) or j (X3) from o0.  Along the normal: faces s in
-// [s0, s1]; tile y covers cells s0-1+(TY-1)y .. s0-2+TY+(TY-1)y.  64 x 8 blocks, two (FP64, 103-118 VGPRs)
-// or three (FP32, 63) per CU: 64 x 10 and 64 x 16 FP32 blocks measured 24 % and 2 %
-// slower, 64 x 4, 64 x 12 and 64 x 16 FP64 blocks 5, 3 and 4 % (192x128x128 torus).
-constexpr int XT_TY = 8;
-template <int DIR, int RECON, int SPEEDS, typename R, typename PT, int GEO, bool PK>
-__global__ void __launch_bounds__(64 * XT_TY, XtOcc<R>::w)
-flux_xt_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> F,
-               R* __restrict__ cmax_out, R* __restrict__ cmin_out, int o0, int no, int s0, int s1,
+template <int RECON, int SPEEDS, typename R, typename PT, int GEO, bool PK>
+__global__ void __launch_bounds__(256, (X1Occ<R, SPEEDS, PK>::w))
+flux_x1_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> F,
+               R* __restrict__ cmax_out, R* __restrict__ cmin_out, int j0, int nj, int k0, int nk,
                const BlockEntry* __restrict__ pk) {
-    constexpr int TY = XT_TY;
-    __shared__ R sr[NV][TY][64];
+    __shared__ R sr[NV][256];
     if constexpr (PK) {
         const long blk = pack_select(pk, b, gd);
         P = pack_at(P, blk * NV * b.nc);
@@ -199,10 +181,22 @@ flux_xt_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> 
         cmax_out = pack_at(cmax_out, blk * 3 * b.nc);
         cmin_out = pack_at(cmin_out, blk * 3 * b.nc);
     }
+    x1_tile<RECON, SPEEDS, R, PT, GEO>(b, c, gd, P, F, cmax_out, cmin_out, j0, nj, k0, nk, blockIdx.x, threadIdx.x, sr);
+}
+
+// X2 / X3 faces.  Transverse columns: flattened (outer, i) with i in [is-1, ie+1]
+// fastest; outer = k (X2) or j (X3) from o0.  Along the normal: faces s in
+// [s0, s1]; tile y covers cells s0-1+(TY-1)y .. s0-2+TY+(TY-1)y.  64 x 8 blocks, two (FP64, 103-118 VGPRs)
+// or three (FP32, 63) per CU: 64 x 10 and 64 x 16 FP32 blocks measured 24 % and 2 %
+// slower, 64 x 4, 64 x 12 and 64 x 16 FP64 blocks 5, 3 and 4 % (192x128x128 torus).
+constexpr int XT_TY = 8;
+template <int DIR, int RECON, int SPEEDS, typename R, typename PT, int GEO, int TY>
+__device__ __forceinline__ void xt_tile(const BlockDims& b, const StepConsts& c, const GeomDev& gd, const Vars<const PT>& P,
+                                        const Vars<R>& F, R* __restrict__ cmax_out, R* __restrict__ cmin_out, int o0,
+                                        int no, int s0, int s1, int bx, int by, int tx, int ty, R (*sr)[TY][64]) {
     const int ni = b.nx1 + 2;
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    const int col = blockIdx.x * 64 + tx;
-    const int s = s0 - 1 + (int)blockIdx.y * (TY - 1) + ty;
+    const int col = bx * 64 + tx;
+    const int s = s0 - 1 + by * (TY - 1) + ty;
     const bool valid = col < ni * no && s <= s1;
     const long st = (DIR == 2) ? b.s2 : b.s3;
     long ci = 0;
@@ -237,6 +231,52 @@ flux_xt_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> 
 #pragma unroll
     for (int v = 0; v < NV; ++v) Pl[v] = sr[v][ty - 1][tx];
     face_flux<DIR, SPEEDS, R, GEO>(c, b, gd, jf, if_, Pl, lo, ci, F, cmax_out, cmin_out);
+}
+template <int DIR, int RECON, int SPEEDS, typename R, typename PT, int GEO, bool PK>
+__global__ void __launch_bounds__(64 * XT_TY, XtOcc<R>::w)
+flux_xt_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> F,
+               R* __restrict__ cmax_out, R* __restrict__ cmin_out, int o0, int no, int s0, int s1,
+               const BlockEntry* __restrict__ pk) {
+    __shared__ R sr[NV][XT_TY][64];
+    if constexpr (PK) {
+        const long blk = pack_select(pk, b, gd);
+        P = pack_at(P, blk * NV * b.nc);
+        F = pack_at(F, blk * 3 * NV * b.nc);
+        cmax_out = pack_at(cmax_out, blk * 3 * b.nc);
+        cmin_out = pack_at(cmin_out, blk * 3 * b.nc);
+    }
+    xt_tile<DIR, RECON, SPEEDS, R, PT, GEO, XT_TY>(b, c, gd, P, F, cmax_out, cmin_out, o0, no, s0, s1, (int)blockIdx.x,
+                                                   (int)blockIdx.y, (int)threadIdx.x, (int)threadIdx.y, sr);
+}
+
+// The faces of all directions in one launch, the X1 tiles first, then X2 and X3
+// tiles of 64 x 4.  A direction's launch of a small block fills a fraction of the
+// chip (64^2: 17 and 20 work-groups on 256 CUs) and ends in a tail that nothing
+// follows; in one launch the directions fill each other's tails, and the smaller
+// X2 / X3 tiles shorten the longest chain.  FP64 64^2: 18.9 + 6.3 -> 11.2 us, 256^2 8.9 +
+// 9 -> 13.5 us, 256x128 torus 10 + 8.1 -> 11.6 us; FP32 128^2 6.8 + 6.1 -> 7.5 us.
+constexpr int ALL_TY = 4;
+// One direction's tiles: its first tile, tiles along the columns, and the face ranges.
+struct FluxTiles { int first, nx, o0, no, s0, s1; };
+template <int RECON, int SPEEDS, typename R, typename PT, int GEO>
+__global__ void __launch_bounds__(256, XtOcc<R>::w)
+flux_all_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> F, R* __restrict__ ctop, FluxTiles x1,
+                  FluxTiles x2, FluxTiles x3) {
+    __shared__ R sr[NV][256];
+    R (*st)[ALL_TY][64] = reinterpret_cast<R (*)[ALL_TY][64]>(sr);
+    const int t = (int)blockIdx.x, tx = (int)threadIdx.x % 64, ty = (int)threadIdx.x / 64;
+    if (t >= x3.first) {
+        const int q = t - x3.first;
+        xt_tile<3, RECON, SPEEDS, R, PT, GEO, ALL_TY>(b, c, gd, P, pack_at(F, 2 * NV * b.nc), pack_at(ctop, 2 * b.nc), nullptr,
+                                                     x3.o0, x3.no, x3.s0, x3.s1, q % x3.nx, q / x3.nx, tx, ty, st);
+    } else if (t >= x2.first) {
+        const int q = t - x2.first;
+        xt_tile<2, RECON, SPEEDS, R, PT, GEO, ALL_TY>(b, c, gd, P, pack_at(F, NV * b.nc), pack_at(ctop, b.nc), nullptr,
+                                                     x2.o0, x2.no, x2.s0, x2.s1, q % x2.nx, q / x2.nx, tx, ty, st);
+    } else {
+        x1_tile<RECON, SPEEDS, R, PT, GEO>(b, c, gd, P, F, ctop, nullptr, x1.o0, x1.no, x1.s0, x1.s1 - x1.s0 + 1, (unsigned)t,
+                                           (int)threadIdx.x, sr);
+    }
 }
 
 // ---------------------------------------------------- FP64, large 3-D blocks
@@ -641,6 +681,73 @@ hipError_t launch_flux_stage(const BlockDims& b, const StepConsts& c, const Geom
                                          (float*)ctop, nullptr, s);
     return launch_prec<double, double>(b, c, gd, dir, recon, speeds, vars_of(P, b.nc), vars_of((double*)F, b.nc),
                                        (double*)ctop, nullptr, s);
+}
+
+// Tiles up to which the directions run in one launch.  Steps of a block, one launch a
+// direction against one: FP64 64^2 82 / 53 us, 256^2 75 / 66, 512^2 135 / 128, 1024^2
+// 433 / 431, 64^3 flat 212 / 195, 1024x512 torus 431 / 416; FP32 fluxes 64^3 flat 173 / 156,
+// 128^3 (31500 tiles) 1004 / 992, 192x128x128 torus (46400 tiles) 1820 / 1837: there the
+// 64 x 8 tiles' fewer overlapping cells win.  FP64 3-D blocks from the size of the
+// marching kernels on take those.
+constexpr long ALL_TILES = 32768;
+// Tiles of the one-launch form, all directions; 0 where a direction is missing.
+static int all_tiles(const BlockDims& b, FluxTiles (&x)[3]) {
+    const int jlo = (b.ndim > 1) ? b.js - 1 : b.js, jhi = (b.ndim > 1) ? b.je + 1 : b.je;
+    const int klo = (b.ndim > 2) ? b.ks - 1 : b.ks, khi = (b.ndim > 2) ? b.ke + 1 : b.ke;
+    const long ni = b.nx1 + 2;
+    const long n1 = (ni * (jhi - jlo + 1) * (khi - klo + 1) - 1 + 254) / 255;
+    x[0] = {0, 0, jlo, jhi - jlo + 1, klo, khi};
+    x[1] = {0, (int)((ni * (khi - klo + 1) + 63) / 64), klo, khi - klo + 1, b.js, b.je + 1};
+    x[2] = {0, (int)((ni * (jhi - jlo + 1) + 63) / 64), jlo, jhi - jlo + 1, b.ks, b.ke + 1};
+    const long n2 = b.ndim > 1 ? (long)x[1].nx * ((b.nx2 + 1 + ALL_TY - 2) / (ALL_TY - 1)) : 0;
+    const long n3 = b.ndim > 2 ? (long)x[2].nx * ((b.nx3 + 1 + ALL_TY - 2) / (ALL_TY - 1)) : 0;
+    const long n = n1 + n2 + n3;
+    if (n > ALL_TILES) return 0;
+    x[1].first = (int)n1;
+    x[2].first = (int)(n1 + n2);
+    return (int)n;
+}
+template <int SPEEDS, typename R, int GEO>
+static hipError_t launch_all(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int recon, const Vars<const R>& P,
+                               const Vars<R>& F, R* ctop, const FluxTiles (&x)[3], int n, hipStream_t s) {
+#define KH_ALL(RECON) \
+    hipLaunchKernelGGL((flux_all_kernel<RECON, SPEEDS, R, R, GEO>), dim3((unsigned)n), dim3(256), 0, s, b, c, gd, P, F, ctop, x[0], x[1], x[2])
+    switch (recon) {
+    case RECON_DONOR: KH_ALL(RECON_DONOR); break;
+    case RECON_LINEAR_MC: KH_ALL(RECON_LINEAR_MC); break;
+    case RECON_PPM: KH_ALL(RECON_PPM); break;
+    default: KH_ALL(RECON_WENO5);
+    }
+#undef KH_ALL
+    return hipGetLastError();
+}
+template <typename R>
+static hipError_t launch_all_prec(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int recon, int speeds,
+                                    const R* P, R* F, R* ctop, const FluxTiles (&x)[3], int n, hipStream_t s) {
+    const Vars<const R> Pv = vars_of(P, b.nc);
+    const Vars<R> Fv = vars_of(F, b.nc);
+    if (b.geo)
+        return speeds == SPEEDS_CTOP ? launch_all<SPEEDS_CTOP, R, 1>(b, c, gd, recon, Pv, Fv, ctop, x, n, s)
+                                     : launch_all<SPEEDS_NONE, R, 1>(b, c, gd, recon, Pv, Fv, ctop, x, n, s);
+    return speeds == SPEEDS_CTOP ? launch_all<SPEEDS_CTOP, R, 0>(b, c, gd, recon, Pv, Fv, ctop, x, n, s)
+                                 : launch_all<SPEEDS_NONE, R, 0>(b, c, gd, recon, Pv, Fv, ctop, x, n, s);
+}
+hipError_t launch_flux_stage_all(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int recon, int prec,
+                                 int speeds, const double* P, const float* P32, void* F, void* ctop, hipStream_t s) {
+    FluxTiles x[3];
+    const bool march = prec == PREC_FP64 && b.ndim > 2 && march_xt(b, (long)(b.nx1 + 2) * (b.nx3 + 2), b.nx2 + 1, 1);
+    const int n = (speeds == SPEEDS_BOTH || march) ? 0 : all_tiles(b, x);
+    if (n)
+        return prec == PREC_SPLIT
+                   ? launch_all_prec<float>(b, c, gd, recon, speeds, P32, (float*)F, (float*)ctop, x, n, s)
+                   : launch_all_prec<double>(b, c, gd, recon, speeds, P, (double*)F, (double*)ctop, x, n, s);
+    const long e = prec == PREC_SPLIT ? sizeof(float) : sizeof(double);
+    for (int dir = 1; dir <= b.ndim; ++dir) {
+        const hipError_t r = launch_flux_stage(b, c, gd, dir, recon, prec, speeds, P, P32, (char*)F + e * (dir - 1) * NV * b.nc,
+                                               (char*)ctop + e * (dir - 1) * b.nc, s, nullptr);
+        if (r != hipSuccess) return r;
+    }
+    return hipSuccess;
 }
 
 // ---------------------------------------------- first-order flux correction

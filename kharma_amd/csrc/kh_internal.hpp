@@ -223,6 +223,10 @@ hipError_t launch_flux(const BlockDims& b, const StepConsts& c, const GeomDev& g
 hipError_t launch_flux_stage(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, int recon, int prec,
                              int speeds, const double* P, const float* P32, void* F, void* ctop, hipStream_t s,
                              const Pack* pk = nullptr);
+// The same for every direction: F [3][8][nc] and ctop [3][nc], in one launch for a
+// small block.
+hipError_t launch_flux_stage_all(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int recon, int prec,
+                                 int speeds, const double* P, const float* P32, void* F, void* ctop, hipStream_t s);
 
 // ---- launchers (kh_step.hip) ----
 hipError_t launch_emf(const BlockDims& b, int prec, const FluxVars<void>& F, void* emf, hipStream_t s);
