@@ -37,10 +37,10 @@ def _torus(n, **kw):
 
 CASES = {
     "mode_weno5": lambda: _mode((81, 83, 79)),
-    "mode_hlle_ppm_ng3": lambda: _mode((127, 65, 66), riemann="hlle", recon="ppm", ng=3),
+    "mode_hlle_ppm_ng3": lambda: _mode((127, 65, 66), riemann="hlle", recon="ppm"),
     "torus_x2_x3": lambda: _torus((97, 74, 73)),
     "torus_x1": lambda: _torus((145, 89, 86)),
-    "torus_x1_ng3": lambda: _torus((121, 101, 90), ng=3),
+    "torus_x1_ng3": lambda: _torus((121, 101, 90)),
 }
 
 
@@ -57,6 +57,10 @@ def test_marching_fluxes_match_the_oracle(oracle_lib, case):
         P = P * (1 + 1e-2 * pr.periodic_fill(rng.uniform(-1, 1, P.shape), cfg))
     ob.init_state(P)
     P, _ = ob.state()
+    ocfg = cfg
+    if case.endswith("ng3"):   # the oracle's faces reach one further and keep four ghosts
+        cfg = dict(cfg, ng=3)
+        P = P[:, 1:-1, 1:-1, 1:-1]
     blk = kh.Block(cfg)
     F, cmax, cmin = blk.new_fluxes()
     Pg = torch.from_numpy(np.ascontiguousarray(P)).cuda()
@@ -67,13 +71,13 @@ def test_marching_fluxes_match_the_oracle(oracle_lib, case):
     torch.cuda.synchronize()
     Fo_all, speeds = ob.array(0), ((cmax.cpu().numpy(), ob.array(1)), (cmin.cpu().numpy(), ob.array(2)))
     for d in (1, 2, 3):
-        sl = face_slices(cfg, d)
-        Fo = Fo_all[d - 1]
+        sl, so = face_slices(cfg, d), face_slices(ocfg, d)
+        Fo = Fo_all[d - 1][(slice(None),) + so]
         Fg = F[d - 1].cpu().numpy()
-        err = np.abs(Fg[(slice(None),) + sl] - Fo[(slice(None),) + sl]).max()
-        assert err <= bar * np.abs(Fo[(slice(None),) + sl]).max(), (case, d, err)
+        err = np.abs(Fg[(slice(None),) + sl] - Fo).max()
+        assert err <= bar * np.abs(Fo).max(), (case, d, err)
         for g, o in speeds:
-            assert np.abs(g[d - 1][sl] - o[d - 1][sl]).max() <= bar * np.abs(o[d - 1][sl]).max(), (case, d)
+            assert np.abs(g[d - 1][sl] - o[d - 1][so]).max() <= bar * np.abs(o[d - 1][so]).max(), (case, d)
         # nothing is written outside the faces the step consumes
         mask = np.ones(Fg.shape[1:], dtype=bool)
         mask[sl] = False
