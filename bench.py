@@ -110,20 +110,17 @@ def _valu_fractions(tag):
     counter summary (profiles/valu_<workload>.json): VALU instructions issued as
     a fraction of the chip's issue capacity (one wave64 instruction per SIMD per
     4 cycles, which for FP64 FMA is the 78.6 TFLOP/s vector peak) and the share
-    of the resident waves' cycles spent waiting on memory.  The update pair is
-    weighted by the kernels' times."""
+    of the resident waves' cycles spent waiting on memory."""
     f = os.path.join(ROOT, "profiles", f"valu_{tag}.json")
     if not os.path.exists(f):
         return None
     k = json.load(open(f))["kernels"]["split"]
     out = {"peak": "78.6 TFLOP/s FP64 vector (VALU issue capacity)", "source": os.path.relpath(f, ROOT)}
-    for ro in ("combine_s2", "recover_s2", "flux_x1_s2", "flux_x2_s2", "flux_x3_s2"):
+    for ro in ("update_s2", "flux_x1_s2", "flux_x2_s2", "flux_x3_s2"):
         if ro in k:
             out[ro] = {"valu_issue_frac": k[ro]["valu_issue_frac"], "wait_frac": k[ro]["wait_any_per_wave_cycle"]}
-    if "combine_s2" in k and "recover_s2" in k:
-        a, b = k["combine_s2"], k["recover_s2"]
-        ta, tb = a["avg_us_under_counters"], b["avg_us_under_counters"]
-        out["update_s2_valu_issue_frac"] = (a["valu_issue_frac"] * ta + b["valu_issue_frac"] * tb) / (ta + tb)
+    if "update_s2" in k:
+        out["update_s2_valu_issue_frac"] = k["update_s2"]["valu_issue_frac"]
     return out
 
 
