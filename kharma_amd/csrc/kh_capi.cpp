@@ -114,6 +114,7 @@ void kh::make_dims(const kh_params* p, BlockDims& b) {
     b.ndim = (p->nx3 > 1) ? 3 : ((p->nx2 > 1) ? 2 : 1);
     b.ng = p->ng;
     b.nx1 = p->nx1; b.nx2 = p->nx2; b.nx3 = p->nx3;
+    b.mesh_nx[0] = p->nx1; b.mesh_nx[1] = p->nx2; b.mesh_nx[2] = p->nx3;
     b.n1 = p->nx1 + 2 * p->ng;
     b.n2 = (b.ndim > 1) ? p->nx2 + 2 * p->ng : 1;
     b.n3 = (b.ndim > 2) ? p->nx3 + 2 * p->ng : 1;
@@ -341,6 +342,7 @@ int kh::block_create_in_mesh(const kh_params* mesh, const int nb[3], const int b
     b->p = pb;
     BlockDims& bd = b->dims;
     fill_dims(&pb, bd);
+    bd.mesh_nx[0] = mesh->nx1; bd.mesh_nx[1] = mesh->nx2; bd.mesh_nx[2] = mesh->nx3;
     bd.dx1 = (mesh->x1max - mesh->x1min) / mesh->nx1;
     bd.dx2 = (mesh->x2max - mesh->x2min) / mesh->nx2;
     bd.dx3 = (mesh->x3max - mesh->x3min) / mesh->nx3;

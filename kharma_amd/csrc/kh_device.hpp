@@ -237,7 +237,10 @@ __device__ __forceinline__ void weno5_cell(float x1, float x2, float x3, float x
 // written as x3 + a / 8 +- b / 4 (a the stencil's second difference, b / 2 its
 // derivative at x3), the weights unnormalised and the sum divided once.  Rounding
 // differs from weno5_cell by an ulp or two (1e-16 of the fluxes, as far from the
-// exact value as weno5_cell).
+// exact value as weno5_cell).  The inversion turns that into 1e-9 of a recovered
+// velocity in zones at the density floor, so the kernels that are not bound by these
+// operations (the tiles, and everything in 2-D) keep weno5_cell, and with it the bits
+// that their states and gradients are compared at.
 __device__ __forceinline__ void weno5_cell_lean(double x1, double x2, double x3, double x4, double x5,
                                                 double& lout, double& rout) {
     constexpr double EPS4 = 4.e-26;

@@ -304,6 +304,8 @@ flux_all_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R>
 //
 // LaneGeom: one lane's metric in LDS, components the flux needs, [MG_N][256].
 enum { MG_G00, MG_G01, MG_G03, MG_G11, MG_G12, MG_G13, MG_G22, MG_G33, MG_U00, MG_U01, MG_U02, MG_U03, MG_UDD, MG_GDET, MG_ALPHA, MG_RF, MG_UF, MG_N };
+// The marching kernels' reconstruction: WENO5 in its lean form (X2 172 -> 165 us, X3 154 ->
+// 144, X1 171 -> 160 on the 192x128x128 torus), which rounds differently from the tiles'.
 template <int RECON>
 __device__ __forceinline__ void march_states(double x1, double x2, double x3, double x4, double x5, double& lout, double& rout) {
     if constexpr (RECON == RECON_WENO5) weno5_cell_lean(x1, x2, x3, x4, x5, lout, rout);
@@ -534,32 +536,36 @@ flux_x1_march_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const double> P
     }
 }
 
-// Rows per resident lane from which the marching kernels are used: two wavefronts
-// per SIMD, 131072 lanes.  A walk pays its start (five rows of loads, one extra
+// Zones per resident lane (two wavefronts per SIMD, 131072 lanes) from which the
+// marching kernels are used.  A walk pays its start (five rows of loads, one extra
 // reconstruction) once per chunk, and two wavefronts hide less latency than the
-// tiles' four, so short walks lose.  Measured, tiles against marching, us: X2/X3
-// 64^3 flat 22 / 25, 99x66x50 torus 32 / 33, 126x90x61 torus 57 / 51, 96^3 flat 64 / 56,
-// 128^3 flat 140 / 111, 192x128x128 torus 246 / 184 and 235 / 163; X1 126x90x61 torus
-// 49 / 52, 192x96x64 81 / 79, 150x110x100 111 / 105, 192x128x128 210 / 180; X1 flat 128^3
-// 112 / 118 (four wavefronts of 103 registers: the tiles stay).  (2-D blocks have one
-// row of each along x3 and too few faces: tiles.)
+// tiles' four, so short walks lose.
+//
+// The zones counted are the whole mesh's, not the launch's: the two families round
+// differently (see march_states), and one block, blocks in one launch and blocks
+// launched one by one give the same bits only if they take the same one.
+//
+// Measured, tiles against marching, us: X2/X3 64^3 flat 22 / 25, 99x66x50 torus 32 / 33,
+// 126x90x61 torus 57 / 51, 96^3 flat 64 / 56, 128^3 flat 140 / 111, 192x128x128 torus 246 /
+// 184 and 235 / 163; X1 126x90x61 torus 49 / 52, 192x96x64 81 / 79, 150x110x100 111 / 105,
+// 192x128x128 210 / 180; X1 flat 128^3 112 / 118 (four wavefronts of 103 registers: the
+// tiles stay).  (2-D blocks have one row of each along x3 and too few faces: tiles.)
 constexpr long MARCH_LANES = 2L * 4 * 256 * 64;
-static bool march_xt(const BlockDims& b, long cols, int nfaces, int nblk) {
-    return b.ndim == 3 && cols * nfaces * nblk >= 4 * MARCH_LANES;
-}
-static bool march_x1(const BlockDims& b, long cells, int nblk) {
-    return b.geo && b.ndim == 3 && cells * nblk >= 8 * MARCH_LANES;
-}
+static long mesh_zones(const BlockDims& b) { return (long)b.mesh_nx[0] * b.mesh_nx[1] * b.mesh_nx[2]; }
+static bool march_xt(const BlockDims& b) { return b.ndim == 3 && mesh_zones(b) >= 4 * MARCH_LANES; }
+static bool march_x1(const BlockDims& b) { return b.geo && b.ndim == 3 && mesh_zones(b) >= 8 * MARCH_LANES; }
 // Faces per chunk: the fewest rounds of work for the busiest CU, a round being one
-// block's chunk plus its start (0.6 of a row's work); a CU holds two blocks, and
-// one alone on it runs at 0.6 of their rate.
+// block's chunk plus its start, 0.6 of a row's work (flat 160^3, X2: chunks of 1, 2, 4, 22
+// faces 299, 233, 193, 171 us); a CU holds two blocks, and one alone on it takes 0.6 of
+// the time of a pair (flat 64x64x32, X2: 198 blocks of 3 faces 15.1 us, 297 of 2 18.2, 585
+// of 1 19.0).
 static int march_chunk(long blocks_x, int nfaces) {
     int best = nfaces;
     double cost = 1e300;
     for (int ch = 1; ch <= nfaces; ++ch) {
         const long blocks = blocks_x * ((nfaces + ch - 1) / ch);
         const double per_cu = (double)((blocks + 255) / 256);
-        const double t = (per_cu > 1.6 ? per_cu : 1.6) * (ch + 0.6);
+        const double t = (per_cu > 1.2 ? per_cu : 1.2) * (ch + 0.6);
         if (t < cost) { cost = t; best = ch; }
     }
     return best;
@@ -578,7 +584,7 @@ static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const Ge
         if (dir == 1) {
             const int nj = jhi - jlo + 1, nk = khi - klo + 1;
             const long cells = (long)(b.nx1 + 6) * nj;
-            if (march_x1(b, cells * nk, nblk)) {
+            if (march_x1(b)) {
                 const unsigned bx = (unsigned)((cells + 4 * 63 - 1) / (4 * 63));
                 const int chunk = march_chunk((long)bx * nblk, nk);
                 const dim3 grid = pack_grid(dim3(bx, (unsigned)((nk + chunk - 1) / chunk)), pk);
@@ -590,7 +596,7 @@ static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const Ge
             const int s0 = dir == 2 ? b.js : b.ks, s1 = dir == 2 ? b.je + 1 : b.ke + 1;
             const long cols = (long)(b.nx1 + 2) * no;
             const int nfaces = s1 - s0 + 1;
-            if (march_xt(b, cols, nfaces, nblk)) {
+            if (march_xt(b)) {
                 const unsigned bx = (unsigned)((cols + 255) / 256);
                 const int chunk = march_chunk((long)bx * nblk, nfaces);
                 const dim3 grid = pack_grid(dim3(bx, (unsigned)((nfaces + chunk - 1) / chunk)), pk);
@@ -735,7 +741,7 @@ static hipError_t launch_all_prec(const BlockDims& b, const StepConsts& c, const
 hipError_t launch_flux_stage_all(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int recon, int prec,
                                  int speeds, const double* P, const float* P32, void* F, void* ctop, hipStream_t s) {
     FluxTiles x[3];
-    const bool march = prec == PREC_FP64 && b.ndim > 2 && march_xt(b, (long)(b.nx1 + 2) * (b.nx3 + 2), b.nx2 + 1, 1);
+    const bool march = prec == PREC_FP64 && march_xt(b);
     const int n = (speeds == SPEEDS_BOTH || march) ? 0 : all_tiles(b, x);
     if (n)
         return prec == PREC_SPLIT

@@ -42,6 +42,7 @@ struct BlockDims {
     // Interior offset of this block in the mesh (zones per axis); coordinates are
     // x = xmin(mesh) + (i - is + goff + 1/2) dx with the mesh's dx.
     int goff[3];
+    int mesh_nx[3];        // interior zones of the whole mesh (the block's own where it is the mesh)
     // Face-centred constrained transport (B_CT): face and edge arrays are
     // [3][n3+1][n2+1][n1+1], index (k fs3 + j fs2 + i) for the lower face / edge of
     // cell (k, j, i), component stride nf.
