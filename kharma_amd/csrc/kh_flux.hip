@@ -545,14 +545,17 @@ flux_x1_march_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const double> P
 // differently (see march_states), and one block, blocks in one launch and blocks
 // launched one by one give the same bits only if they take the same one.
 //
-// Measured, tiles against marching, us: X2/X3 64^3 flat 22 / 25, 99x66x50 torus 32 / 33,
-// 126x90x61 torus 57 / 51, 96^3 flat 64 / 56, 128^3 flat 140 / 111, 192x128x128 torus 246 /
-// 184 and 235 / 163; X1 126x90x61 torus 49 / 52, 192x96x64 81 / 79, 150x110x100 111 / 105,
+// FP64 steps, the tiles in one launch (flux_all_kernel) against marching, us: flat 80^3
+// 322 / 350, 96^3 541 / 544, 112^3 835 / 797, 128^3 1259 / 1132 (7 zones a lane: 97^3);
+// torus 84x72x60 313 / 345, 102x84x66 475 / 494, 126x90x61 537 / 547, 128x96x96 869 / 839,
+// 160x112x96 1270 / 1171.  The task entry points, which launch a direction at a time, gain
+// earlier (126x90x61, X2/X3 a face launch 57 / 51 us), so curved space starts at 5.  X1,
+// curved space only: 126x90x61 49 / 52 us, 192x96x64 81 / 79, 150x110x100 111 / 105,
 // 192x128x128 210 / 180; X1 flat 128^3 112 / 118 (four wavefronts of 103 registers: the
 // tiles stay).  (2-D blocks have one row of each along x3 and too few faces: tiles.)
 constexpr long MARCH_LANES = 2L * 4 * 256 * 64;
 static long mesh_zones(const BlockDims& b) { return (long)b.mesh_nx[0] * b.mesh_nx[1] * b.mesh_nx[2]; }
-static bool march_xt(const BlockDims& b) { return b.ndim == 3 && mesh_zones(b) >= 4 * MARCH_LANES; }
+static bool march_xt(const BlockDims& b) { return b.ndim == 3 && mesh_zones(b) >= (b.geo ? 5 : 7) * MARCH_LANES; }
 static bool march_x1(const BlockDims& b) { return b.geo && b.ndim == 3 && mesh_zones(b) >= 8 * MARCH_LANES; }
 // Faces per chunk: the fewest rounds of work for the busiest CU, a round being one
 // block's chunk plus its start, 0.6 of a row's work (flat 160^3, X2: chunks of 1, 2, 4, 22
