@@ -19,7 +19,7 @@ INCLUDE = os.path.abspath(os.path.join(HERE, "..", "include"))
 SOURCES = ["kh_flux.hip", "kh_step.hip", "kh_update.hip", "kh_update_f32.hip",
            "kh_update_f64.hip", "kh_adjoint.hip", "kh_mesh.hip", "kh_ct.hip", "kh_capi.cpp", "kh_adjoint_capi.cpp",
            "kh_mesh_capi.cpp", "kh_geom.cpp", "kh_problem.cpp"]
-HEADERS = ["kh_device.hpp", "kh_step.hpp", "kh_update_geo.hpp", "kh_adjoint.hpp", "kh_internal.hpp", "kh_host.hpp"]
+HEADERS = ["kh_device.hpp", "kh_lane_geom.hpp", "kh_step.hpp", "kh_update_geo.hpp", "kh_adjoint.hpp", "kh_internal.hpp", "kh_host.hpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("KH_OFFLOAD_ARCH", "gfx950")

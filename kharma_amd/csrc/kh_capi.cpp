@@ -211,6 +211,10 @@ hipError_t upload_geometry(kh_block* b) {
         if (e != hipSuccess) return e;
         d.g32[loc] = (const float*)q;
     }
+    d.lane_form = true;
+    for (int loc = 0; loc < 3; ++loc)
+        for (int comp : {2, 8})
+            for (long q = 0; q < G.np; ++q) d.lane_form &= G.g[loc][(size_t)comp * G.np + q] == 0.;
     unsigned long long mask = 0;
     for (int n = 0; n < 64; ++n)
         for (long q = 0; q < G.np; ++q)

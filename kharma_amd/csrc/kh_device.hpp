@@ -402,6 +402,10 @@ __device__ __forceinline__ void prim_to_u_and_flux(const G& g, const R P[NV], co
     }
 }
 
+// g^{ab} of a metric, the component named at compile time (overloaded for a metric
+// that holds some of them only).
+template <int A, int B, class G> __device__ __forceinline__ auto gcon_at(const G& g) { return g.gcon(A, B); }
+
 // Flux::vchar, flux_functions.hpp:368-439 (the two clip() calls there are no-ops,
 // so cs2 and cms2 are deliberately left unclamped here too).
 template <typename R, class G, int DIR>
@@ -418,7 +422,7 @@ __device__ __forceinline__ void vchar(const G& g, const R P[NV], const FourVec<R
         B = R(2) * (Au * Bu - (Au * Bu) * cms2);
         C = Au * Au - (R(1) + Au * Au) * cms2;
     } else {
-        const R Asq = g.gcon(DIR, DIR), Bsq = g.gcon(0, 0), AB = g.gcon(0, DIR);
+        const R Asq = gcon_at<DIR, DIR>(g), Bsq = gcon_at<0, 0>(g), AB = gcon_at<0, DIR>(g);
         const R Au = D.ucon[DIR], Bu = D.ucon[0];
         A = Bu * Bu - (Bsq + Bu * Bu) * cms2;
         B = R(2) * (Au * Bu - (AB + Au * Bu) * cms2);

@@ -15,6 +15,7 @@
 // a wavefront reads 64 consecutive values), y walks TY cells along the face
 // normal, consecutive tiles overlapping by one cell.
 #include "kh_internal.hpp"
+#include "kh_lane_geom.hpp"
 
 namespace kh {
 
@@ -302,8 +303,6 @@ flux_all_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R>
 // (249 us X2: the metric's waits included the prefetch) and the metric straight
 // from memory behind it (250 us X2, 182 us X3) were slower.
 //
-// LaneGeom: one lane's metric in LDS, components the flux needs, [MG_N][256].
-enum { MG_G00, MG_G01, MG_G03, MG_G11, MG_G12, MG_G13, MG_G22, MG_G33, MG_U00, MG_U01, MG_U02, MG_U03, MG_UDD, MG_GDET, MG_ALPHA, MG_RF, MG_UF, MG_N };
 // The marching kernels' reconstruction: WENO5 in its lean form (X2 172 -> 165 us, X3 154 ->
 // 144, X1 171 -> 160 on the 192x128x128 torus), which rounds differently from the tiles'.
 template <int RECON>
@@ -311,39 +310,6 @@ __device__ __forceinline__ void march_states(double x1, double x2, double x3, do
     if constexpr (RECON == RECON_WENO5) weno5_cell_lean(x1, x2, x3, x4, x5, lout, rout);
     else cell_states<RECON, double>(x1, x2, x3, x4, x5, lout, rout);
 }
-template <int DIR> struct LaneGeom {
-    static constexpr bool flat = false;
-    const double (*s)[256];
-    int t;
-    static __device__ __forceinline__ constexpr int src(int m) {   // component of the cached table
-        return m == MG_G00 ? 0 : m == MG_G01 ? 1 : m == MG_G03 ? 3 : m == MG_G11 ? 4 : m == MG_G12 ? 5 : m == MG_G13 ? 6
-             : m == MG_G22 ? 7 : m == MG_G33 ? 9 : m == MG_U00 ? 10 : m == MG_U01 ? 11 : m == MG_U02 ? 12 : m == MG_U03 ? 13
-             : m == MG_UDD ? (DIR == 1 ? 14 : DIR == 2 ? 17 : 19) : m == MG_GDET ? GEO_GDET : GEO_ALPHA;
-    }
-    __device__ __forceinline__ double gcov(int a, int b) const {
-        const int l = a < b ? a : b, h = a < b ? b : a;
-        return s[l == 0 ? (h == 0 ? MG_G00 : h == 1 ? MG_G01 : MG_G03)
-               : l == 1 ? (h == 1 ? MG_G11 : h == 2 ? MG_G12 : MG_G13) : l == 2 ? MG_G22 : MG_G33][t];
-    }
-    __device__ __forceinline__ double gcon(int a, int b) const {
-        return a == 0 ? s[MG_U00 + b][t] : s[MG_UDD][t];
-    }
-    __device__ __forceinline__ double gcon0(int v) const { return s[MG_U00 + v][t]; }
-    __device__ __forceinline__ double gdet() const { return s[MG_GDET][t]; }
-    __device__ __forceinline__ double alpha() const { return s[MG_ALPHA][t]; }
-    // CachedGeom::lower without the products with g_{t x2} and g_{x2 phi}, which vanish
-    __device__ __forceinline__ void lower(const double v[4], double o[4]) const {
-        o[0] = fma(gcov(0, 3), v[3], fma(gcov(0, 0), v[0], gcov(0, 1) * v[1]));
-        o[1] = sum_a(gcov(0, 1), v[0], gcov(1, 1), v[1], gcov(1, 2), v[2], gcov(1, 3), v[3]);
-        o[2] = fma(gcov(2, 2), v[2], gcov(1, 2) * v[1]);
-        o[3] = fma(gcov(3, 3), v[3], fma(gcov(0, 3), v[0], gcov(1, 3) * v[1]));
-    }
-    __device__ __forceinline__ double lorentz(double u1, double u2, double u3) const {
-        const double qsq = gcov(1, 1) * u1 * u1 + gcov(2, 2) * u2 * u2 + gcov(3, 3) * u3 * u3 +
-                           2. * (gcov(1, 2) * u1 * u2 + gcov(1, 3) * u1 * u3);
-        return sqrt(1. + qsq);
-    }
-};
 template <int DIR, int RECON, int SPEEDS, int GEO, bool PK>
 __global__ void __launch_bounds__(256, 2)
 flux_march_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const double> P, Vars<double> F,
@@ -555,8 +521,12 @@ flux_x1_march_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const double> P
 // tiles stay).  (2-D blocks have one row of each along x3 and too few faces: tiles.)
 constexpr long MARCH_LANES = 2L * 4 * 256 * 64;
 static long mesh_zones(const BlockDims& b) { return (long)b.mesh_nx[0] * b.mesh_nx[1] * b.mesh_nx[2]; }
-static bool march_xt(const BlockDims& b) { return b.ndim == 3 && mesh_zones(b) >= (b.geo ? 5 : 7) * MARCH_LANES; }
-static bool march_x1(const BlockDims& b) { return b.geo && b.ndim == 3 && mesh_zones(b) >= 8 * MARCH_LANES; }
+static bool march_xt(const BlockDims& b, const GeomDev& gd) {
+    return b.ndim == 3 && (b.geo ? gd.lane_form && mesh_zones(b) >= 5 * MARCH_LANES : mesh_zones(b) >= 7 * MARCH_LANES);
+}
+static bool march_x1(const BlockDims& b, const GeomDev& gd) {
+    return b.geo && gd.lane_form && b.ndim == 3 && mesh_zones(b) >= 8 * MARCH_LANES;
+}
 // Faces per chunk: the fewest rounds of work for the busiest CU, a round being one
 // block's chunk plus its start, 0.6 of a row's work (flat 160^3, X2: chunks of 1, 2, 4, 22
 // faces 299, 233, 193, 171 us); a CU holds two blocks, and one alone on it takes 0.6 of
@@ -587,7 +557,7 @@ static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const Ge
         if (dir == 1) {
             const int nj = jhi - jlo + 1, nk = khi - klo + 1;
             const long cells = (long)(b.nx1 + 6) * nj;
-            if (march_x1(b)) {
+            if (march_x1(b, gd)) {
                 const unsigned bx = (unsigned)((cells + 4 * 63 - 1) / (4 * 63));
                 const int chunk = march_chunk((long)bx * nblk, nk);
                 const dim3 grid = pack_grid(dim3(bx, (unsigned)((nk + chunk - 1) / chunk)), pk);
@@ -599,7 +569,7 @@ static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const Ge
             const int s0 = dir == 2 ? b.js : b.ks, s1 = dir == 2 ? b.je + 1 : b.ke + 1;
             const long cols = (long)(b.nx1 + 2) * no;
             const int nfaces = s1 - s0 + 1;
-            if (march_xt(b)) {
+            if (march_xt(b, gd)) {
                 const unsigned bx = (unsigned)((cols + 255) / 256);
                 const int chunk = march_chunk((long)bx * nblk, nfaces);
                 const dim3 grid = pack_grid(dim3(bx, (unsigned)((nfaces + chunk - 1) / chunk)), pk);
@@ -744,7 +714,7 @@ static hipError_t launch_all_prec(const BlockDims& b, const StepConsts& c, const
 hipError_t launch_flux_stage_all(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int recon, int prec,
                                  int speeds, const double* P, const float* P32, void* F, void* ctop, hipStream_t s) {
     FluxTiles x[3];
-    const bool march = prec == PREC_FP64 && march_xt(b);
+    const bool march = prec == PREC_FP64 && march_xt(b, gd);
     const int n = (speeds == SPEEDS_BOTH || march) ? 0 : all_tiles(b, x);
     if (n)
         return prec == PREC_SPLIT

@@ -161,6 +161,7 @@ struct GeomDev {
     const float* flr32 = nullptr;
     int gn1 = 0;
     long np = 0;
+    bool lane_form = false;   // g_{t x2} and g_{x2 phi} are zero at every point (mesh: of every block)
 };
 enum SpeedsOut { SPEEDS_NONE = 0, SPEEDS_BOTH = 1, SPEEDS_CTOP = 2 };
 

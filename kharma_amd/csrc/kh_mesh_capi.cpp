@@ -240,6 +240,9 @@ int kh_mesh_create(const kh_params* p, int nb1, int nb2, int nb3, kh_mesh** out)
             k->geo_bufs.clear();
             k->geo = m->blk[b % (nb1 * nb2)]->geo;
         }
+    bool lane_form = true;   // one answer for the mesh: its blocks run the same kernels
+    for (const kh_block* k : m->blk) lane_form &= k->geo.lane_form;
+    for (kh_block* k : m->blk) k->geo.lane_form = lane_form;
     const BlockDims& bd = m->blk[0]->dims;
     m->n_dt = dt_blocks(bd);
     m->n_divb = divb_blocks(bd);
