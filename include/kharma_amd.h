@@ -410,6 +410,11 @@ int kh_driver_arrays(kh_driver* d, double** U, double** P);
 /* Per-kernel timing with HIP events recorded on the driver's stream around every
  * launch of kh_driver_step while enabled (no counterpart in the reference; it
  * plays the role of the Kokkos-tools kernel timer hooked in run.sh:11-91).
+ * While enabled, each direction's face fluxes are a launch of their own, to be
+ * timed by direction.  With timing off a small block (up to 32768 tiles of 255
+ * X1 cells or of 64 x 3 X2 / X3 faces) runs all directions in one launch, which
+ * takes less than the sum of the three times; the results are the same bit for
+ * bit.
  * Kernel kinds: 0..2 face fluxes X1..X3, 3 physical-boundary flux fixes and ghost fills, 4 stage-1 update,
  * 5 stage-2 update, 6 inversion fix-up, 7 divB, 8 timestep finalize. */
 #define KH_NKERNEL_KINDS 9

@@ -708,6 +708,8 @@ class Driver:
     KERNEL_KINDS = ("flux_x1", "flux_x2", "flux_x3", "bounds", "update_s1", "update_s2", "fixup", "divb", "finalize")
 
     def set_kernel_timing(self, enable):
+        """Time each kernel of step().  While on, the face fluxes run one launch a
+        direction; off, a small block runs them in one launch, with the same results."""
         _check(lib().kh_driver_set_kernel_timing(self.h, int(bool(enable))))
 
     def kernel_times(self):
