@@ -246,7 +246,8 @@ adj_divct_kernel(BlockDims b, const double* __restrict__ ld, double* __restrict_
         }
     }
     if (seed.dir) {
-        // a face-flux objective's seed (adj_seed_kernel's faces, fluid variables)
+        // a face-flux objective's seed: the faces of index `face` along dir, over the interior
+        // transverse range (fluid variables)
         const int k = (int)(x / s3), j = (int)((x - (long)k * s3) / s2), i = (int)(x - (long)k * s3 - (long)j * s2);
         const int along = (seed.dir == 1) ? i : (seed.dir == 2) ? j : k;
         const bool t1 = (seed.dir == 1) || (i >= b.is && i <= b.ie);
@@ -854,22 +855,6 @@ __global__ void __launch_bounds__(ABS) save_x1_flux_kernel(BlockDims b, const do
     x1f[t] = F[RHO * b.nc + (long)k * b.s3 + (long)j * b.s2 + i];
 }
 
-// Adjoint seed of a face-flux objective: lF_dir[var] += w on the faces of
-// index `face` along dir, over the interior transverse range.
-__global__ void __launch_bounds__(ABS) adj_seed_kernel(BlockDims b, int dir, int var, int face, double w,
-                                                       double* __restrict__ lF) {
-    const int na = (dir == 1) ? (b.ndim > 1 ? b.nx2 : 1) : b.nx1;
-    const int nb = (dir == 3) ? (b.ndim > 1 ? b.nx2 : 1) : (b.ndim > 2 ? b.nx3 : 1);
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= na * nb) return;
-    const int ta = t % na, tb = t / na;
-    int i, j, k;
-    if (dir == 1) { i = face; j = b.js + ta; k = b.ks + tb; }
-    else if (dir == 2) { i = b.is + ta; j = face; k = b.ks + tb; }
-    else { i = b.is + ta; k = face; j = b.js + tb; }
-    lF[((long)(dir - 1) * NV + var) * b.nc + (long)k * b.s3 + (long)j * b.s2 + i] += w;
-}
-
 // Transpose of the periodic ghost fill: each interior zone collects the
 // adjoints held by its periodic images (up to 3 per axis offset, corners
 // included); ghosts are cleared by adj_clear_ghosts afterwards.
@@ -1182,13 +1167,6 @@ hipError_t launch_adj_fix_flux(const BlockDims& b, double* lF, const double* x1f
     const long n = npolar + x1_flux_rows(b);
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(adj_fix_flux_kernel, agrid(n), dim3(ABS), 0, s, b, lF, x1f);
-    return hipGetLastError();
-}
-
-hipError_t launch_adj_seed(const BlockDims& b, int dir, int var, int face, double w, double* lF, hipStream_t s) {
-    const int na = (dir == 1) ? (b.ndim > 1 ? b.nx2 : 1) : b.nx1;
-    const int nb = (dir == 3) ? (b.ndim > 1 ? b.nx2 : 1) : (b.ndim > 2 ? b.nx3 : 1);
-    hipLaunchKernelGGL(adj_seed_kernel, agrid((long)na * nb), dim3(ABS), 0, s, b, dir, var, face, w, lF);
     return hipGetLastError();
 }
 

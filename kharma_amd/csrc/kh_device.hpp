@@ -31,7 +31,6 @@ template <class G, typename R> __device__ __forceinline__ R bsq_of(const R b[4],
     if constexpr (G::flat) return dot4(b, c);
     else return fma(b[3], c[3], fma(b[2], c[2], fma(b[0], c[0], b[1] * c[1])));
 }
-template <typename R> __device__ __forceinline__ R dmax(R a, R b) { return a > b ? a : (b != b ? b : a); }
 // std::max / std::min semantics (return the first argument unless the second compares greater/less)
 template <typename R> __device__ __forceinline__ R smax(R a, R b) { return (a < b) ? b : a; }
 template <typename R> __device__ __forceinline__ R smin(R a, R b) { return (b < a) ? b : a; }
@@ -261,46 +260,6 @@ __device__ __forceinline__ void weno5_cell_lean(double x1, double x2, double x3,
 }
 
 // ------------------------------------------------------------ reconstruction
-// WENO5 of Tchekhovskoy+07 / Shu 2011 as in flux/reconstruction.hpp:128-204.
-// The nonlinear weights (c_i / (EPS+beta_i)^2) / sum are evaluated in the
-// equivalent scaled form c_i r_i^2 / sum(c r^2), r_i = min_j(EPS+beta_j)/(EPS+beta_i),
-// which cannot under/overflow in FP32 (EPS^2 = 1e-52 underflows a float).
-template <typename R>
-__device__ __forceinline__ void weno5_beta(R x1, R x2, R x3, R x4, R x5, R t[3]) {
-    constexpr R EPS = R(1.e-26);
-    R c1 = x1 - R(2) * x2 + x3, c2 = x1 - R(4) * x2 + R(3) * x3;
-    t[0] = EPS + (R(13. / 12.) * c1 * c1 + R(0.25) * c2 * c2);
-    c1 = x2 - R(2) * x3 + x4; c2 = x4 - x2;
-    t[1] = EPS + (R(13. / 12.) * c1 * c1 + R(0.25) * c2 * c2);
-    c1 = x3 - R(2) * x4 + x5; c2 = x5 - R(4) * x4 + R(3) * x3;
-    t[2] = EPS + (R(13. / 12.) * c1 * c1 + R(0.25) * c2 * c2);
-}
-// value at the right face of the centre cell (x3)
-template <typename R>
-__device__ __forceinline__ R weno5_right(R x1, R x2, R x3, R x4, R x5) {
-    R t[3];
-    weno5_beta(x1, x2, x3, x4, x5, t);
-    const R tm = smin(smin(t[0], t[1]), t[2]);
-    const R r0 = tm / t[0], r1 = tm / t[1], r2 = tm / t[2];
-    const R w0 = R(1. / 16.) * r0 * r0, w1 = R(5. / 8.) * r1 * r1, w2 = R(5. / 16.) * r2 * r2;
-    const R iW = R(1) / (w0 + w1 + w2);
-    return ((R(3. / 8.) * x1 - R(5. / 4.) * x2 + R(15. / 8.) * x3) * (w0 * iW) +
-            (R(-1. / 8.) * x2 + R(3. / 4.) * x3 + R(3. / 8.) * x4) * (w1 * iW) +
-            (R(3. / 8.) * x3 + R(3. / 4.) * x4 - R(1. / 8.) * x5) * (w2 * iW));
-}
-// value at the left face of the centre cell (x3)
-template <typename R>
-__device__ __forceinline__ R weno5_left(R x1, R x2, R x3, R x4, R x5) {
-    R t[3];
-    weno5_beta(x1, x2, x3, x4, x5, t);
-    const R tm = smin(smin(t[0], t[1]), t[2]);
-    const R r0 = tm / t[0], r1 = tm / t[1], r2 = tm / t[2];
-    const R w0 = R(1. / 16.) * r2 * r2, w1 = R(5. / 8.) * r1 * r1, w2 = R(5. / 16.) * r0 * r0;
-    const R iW = R(1) / (w0 + w1 + w2);
-    return ((R(3. / 8.) * x5 - R(5. / 4.) * x4 + R(15. / 8.) * x3) * (w0 * iW) +
-            (R(-1. / 8.) * x4 + R(3. / 4.) * x3 + R(3. / 8.) * x2) * (w1 * iW) +
-            (R(3. / 8.) * x3 + R(3. / 4.) * x2 - R(1. / 8.) * x1) * (w2 * iW));
-}
 // MC-limited linear (reconstruction.hpp:52-56,107-123)
 template <typename R> __device__ __forceinline__ R mc_lim(R dm, R dp) {
     const R r = (fabs(dp) > R(0) ? dm / dp : R(2));
@@ -324,26 +283,6 @@ __device__ __forceinline__ void ppm(R q_im2, R q_im1, R q_i, R q_ip1, R q_ip2, R
 }
 
 enum Recon { RECON_DONOR = 0, RECON_LINEAR_MC = 1, RECON_WENO5 = 2, RECON_PPM = 3 };
-
-// Face states from a 6-point stencil x[-3..2] around face "0" (left face of cell 0):
-// ql = right edge of cell -1, qr = left edge of cell 0.
-template <int RECON, typename R>
-__device__ __forceinline__ void face_states(const R x[6], R& ql, R& qr) {
-    if constexpr (RECON == RECON_WENO5) {
-        ql = weno5_right(x[0], x[1], x[2], x[3], x[4]);
-        qr = weno5_left(x[1], x[2], x[3], x[4], x[5]);
-    } else if constexpr (RECON == RECON_LINEAR_MC) {
-        ql = x[2] + R(0.5) * (mc_lim(x[2] - x[1], x[3] - x[2]) * (x[3] - x[2]));
-        qr = x[3] - R(0.5) * (mc_lim(x[3] - x[2], x[4] - x[3]) * (x[4] - x[3]));
-    } else if constexpr (RECON == RECON_PPM) {
-        R a, b;
-        ppm(x[0], x[1], x[2], x[3], x[4], a, ql);
-        ppm(x[1], x[2], x[3], x[4], x[5], qr, b);
-    } else {
-        ql = x[2];
-        qr = x[3];
-    }
-}
 
 // ----------------------------------------------------------------- GRMHD
 // GRMHD::calc_4vecs, grmhd/grmhd_functions.hpp:225-246.  U0A: u_t by lower0_a.
@@ -919,13 +858,6 @@ __device__ __forceinline__ double wave_min(double v) {
 __device__ __forceinline__ double wave_max(double v) {
     for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
     return v;
-}
-// Non-negative doubles order like their bit patterns: atomic min/max on u64.
-__device__ __forceinline__ void atomic_min_pos(unsigned long long* addr, double v) {
-    atomicMin(addr, (unsigned long long)__double_as_longlong(v));
-}
-__device__ __forceinline__ void atomic_max_pos(unsigned long long* addr, double v) {
-    atomicMax(addr, (unsigned long long)__double_as_longlong(v));
 }
 
 }  // namespace kh

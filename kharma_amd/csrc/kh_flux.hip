@@ -127,8 +127,7 @@ __device__ __forceinline__ void face_flux(const StepConsts& c, const BlockDims& 
 // 192x128x128 torus) and for the X1 kernels (67-68 instead of 90-115).  The
 // FP64 kernels keep their 140-142 VGPRs: a 4-wave bound spills 28-36 bytes per
 // lane and is slower.
-template <typename R, int SPEEDS, bool PK> struct X1Occ { static constexpr int w = sizeof(R) == 4 ? 6 : 1; };
-template <typename R> struct XtOcc { static constexpr int w = sizeof(R) == 4 ? 6 : 1; };
+template <typename R> struct FluxOcc { static constexpr int w = sizeof(R) == 4 ? 6 : 1; };
 template <int RECON, int SPEEDS, typename R, typename PT, int GEO>
 __device__ __forceinline__ void x1_tile(const BlockDims& b, const StepConsts& c, const GeomDev& gd, const Vars<const PT>& P,
                                         const Vars<R>& F, R* __restrict__ cmax_out, R* __restrict__ cmin_out, int j0,
@@ -170,7 +169,7 @@ __device__ __forceinline__ void x1_tile(const BlockDims& b, const StepConsts& c,
     face_flux<1, SPEEDS, R, GEO>(c, b, gd, jf, b.is - 1 + ii, Pl, lo, ci, F, cmax_out, cmin_out);
 }
 template <int RECON, int SPEEDS, typename R, typename PT, int GEO, bool PK>
-__global__ void __launch_bounds__(256, (X1Occ<R, SPEEDS, PK>::w))
+__global__ void __launch_bounds__(256, FluxOcc<R>::w)
 flux_x1_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> F,
                R* __restrict__ cmax_out, R* __restrict__ cmin_out, int j0, int nj, int k0, int nk,
                const BlockEntry* __restrict__ pk) {
@@ -234,7 +233,7 @@ __device__ __forceinline__ void xt_tile(const BlockDims& b, const StepConsts& c,
     face_flux<DIR, SPEEDS, R, GEO>(c, b, gd, jf, if_, Pl, lo, ci, F, cmax_out, cmin_out);
 }
 template <int DIR, int RECON, int SPEEDS, typename R, typename PT, int GEO, bool PK>
-__global__ void __launch_bounds__(64 * XT_TY, XtOcc<R>::w)
+__global__ void __launch_bounds__(64 * XT_TY, FluxOcc<R>::w)
 flux_xt_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> F,
                R* __restrict__ cmax_out, R* __restrict__ cmin_out, int o0, int no, int s0, int s1,
                const BlockEntry* __restrict__ pk) {
@@ -260,7 +259,7 @@ constexpr int ALL_TY = 4;
 // One direction's tiles: its first tile, tiles along the columns, and the face ranges.
 struct FluxTiles { int first, nx, o0, no, s0, s1; };
 template <int RECON, int SPEEDS, typename R, typename PT, int GEO>
-__global__ void __launch_bounds__(256, XtOcc<R>::w)
+__global__ void __launch_bounds__(256, FluxOcc<R>::w)
 flux_all_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> F, R* __restrict__ ctop, FluxTiles x1,
                   FluxTiles x2, FluxTiles x3) {
     __shared__ R sr[NV][256];

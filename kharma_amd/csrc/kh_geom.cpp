@@ -195,10 +195,6 @@ void native_dxdX(const kh_params& p, const double X[4], double M[4][4]) {
     make_embedding(p).dxdX(X, M);
 }
 
-void native_gcov(const kh_params& p, const double X[4], double g[4][4]) {
-    make_embedding(p).gcov_native(X, g);
-}
-
 double invert_metric(const double g[4][4], double gi[4][4]) { return invert4(g, gi); }
 
 static const int SYM[10][2] = {{0, 0}, {0, 1}, {0, 2}, {0, 3}, {1, 1}, {1, 2}, {1, 3}, {2, 2}, {2, 3}, {3, 3}};

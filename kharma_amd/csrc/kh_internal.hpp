@@ -148,7 +148,6 @@ void locus_coords(const kh_params& p, const BlockDims& b, int loc, int j, int i,
 double embed_r(const kh_params& p, const double X[4]);
 void embed_coords(const kh_params& p, const double X[4], double Xe[4]);
 void native_dxdX(const kh_params& p, const double X[4], double M[4][4]);
-void native_gcov(const kh_params& p, const double X[4], double g[4][4]);
 double invert_metric(const double g[4][4], double gi[4][4]);
 
 // Device copy of the cache.  The flux kernels of the split form read the FP32 copies.
@@ -349,7 +348,6 @@ hipError_t launch_ptou(const BlockDims& b, const StepConsts& c, const GeomDev& g
 // number of variables of a contiguous [nvar][nc] array.
 hipError_t launch_sync(const BlockDims& b, const Vars<double>& A, int nvar, hipStream_t s);
 hipError_t launch_sync(const BlockDims& b, double* A, int nvar, hipStream_t s);
-hipError_t launch_sync_int(const BlockDims& b, int* A, hipStream_t s);
 
 // ---- mesh of several blocks (kh_mesh.hip) ----
 // Extents of a uniform mesh of nb[0] x nb[1] x nb[2] equal blocks: N interior
@@ -411,7 +409,6 @@ hipError_t launch_adj_bounds(const BlockDims& b, const GeomDev& gd, const double
 long x1_flux_rows(const BlockDims& b);
 hipError_t launch_save_x1_flux(const BlockDims& b, const double* F, double* x1f, hipStream_t s);
 hipError_t launch_adj_fix_flux(const BlockDims& b, double* lF, const double* x1f, hipStream_t s);
-hipError_t launch_adj_seed(const BlockDims& b, int dir, int var, int face, double w, double* lF, hipStream_t s);
 hipError_t launch_adj_ptou(const BlockDims& b, const StepConsts& c, const GeomDev& gd, const double* P,
                            const double* lU, double* lP, hipStream_t s);
 hipError_t launch_adj_fold(const BlockDims& b, double* A, int nvar, hipStream_t s);

@@ -1029,10 +1029,6 @@ hipError_t launch_sync(const BlockDims& b, double* A, int nvar, hipStream_t s) {
     }
     return hipSuccess;
 }
-hipError_t launch_sync_int(const BlockDims& b, int* A, hipStream_t s) {
-    hipLaunchKernelGGL(sync_kernel<int>, grid_for(b.nc), dim3(BS), 0, s, b, vars_of(A, b.nc));
-    return hipGetLastError();
-}
 hipError_t launch_estimate_dt(const BlockDims& b, const StepConsts& c, int prec, const void* cmax, const void* cmin,
                               double* part, hipStream_t s) {
     const dim3 g = grid_for(ninterior_host(b));

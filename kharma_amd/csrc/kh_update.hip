@@ -12,12 +12,8 @@
 
 namespace kh {
 
-// Work-groups per CU the update kernel is compiled for: 4 (128 VGPRs) with the
-// flat metric; the cached-metric variant needs ~240 VGPRs and would spill at 4.
-template <int GEO> struct UpdateOcc { static constexpr int min_blocks = GEO ? 2 : 4; };
-
-
-// ------------------------------------------------------- fused stage update
+// --------------------------------------- fused stage update, flat space
+// Compiled for 4 work-groups per CU (128 VGPRs).
 // Stage 1 (gam0 = 0 and U_sub == U_full) reads the state once: 0*U + 1*U == U.
 // ND: the dimensionality where it is known at compile time, else 0.  Known, the
 // fluxes are requested in one go instead of in two parts about a branch, which suits
@@ -27,8 +23,8 @@ template <int GEO> struct UpdateOcc { static constexpr int min_blocks = GEO ? 2 
 // BM: 0 no B transport (1-D), 1 flux-CT EMFs from the face fluxes, 2 face-centred
 // B (B_CT): the cell B is the average of the stage's new faces fB (B_CT::BlockUtoP,
 // b_ct.cpp:173-205, which the reference runs before the inversion).
-template <typename R, bool DO_DT, int ND, int BM, int GEO, int INV = 0, bool PK = false>
-__global__ void __launch_bounds__(BS, UpdateOcc<GEO>::min_blocks)
+template <typename R, bool DO_DT, int ND, int BM, int INV = 0, bool PK = false>
+__global__ void __launch_bounds__(BS, 4)
 update_kernel(BlockDims b, StepConsts cst, GeomDev gd, int stage, const R* __restrict__ F, const R* __restrict__ ctop,
               const double* __restrict__ Usub, const double* Ufull, const double* __restrict__ Psub,
               double* Uout, double* __restrict__ Pout, float* __restrict__ Pout32,
@@ -58,14 +54,6 @@ update_kernel(BlockDims b, StepConsts cst, GeomDev gd, int stage, const R* __res
         double dudt[NV];
         if constexpr (BM == 1) zone_divergence_ct<R, ND>(b, F, c, dudt);
         else zone_divergence<R>(b, flux_vars_of(F, b.nc), nullptr, c, false, dudt, BM == 2);
-        if constexpr (GEO) {
-            double Ps[NV];
-#pragma unroll
-            for (int v = 0; v < NV; ++v) Ps[v] = Psub[v * b.nc + c];
-            const long q = (long)j * gd.gn1 + i;
-            CachedGeom<double> g(gd.g[GLOC_CENTER], gd.np, q);
-            add_geo_source(g, gd, q, Ps, gam, dudt);
-        }
         const double g0 = cst.gam0[stage - 1], g1 = cst.gam1[stage - 1];
         const double beta_dt = cst.beta[stage - 1] * ds->dt;
         const bool same = (g0 == 0.) && (Usub == Ufull);
@@ -87,8 +75,8 @@ update_kernel(BlockDims b, StepConsts cst, GeomDev gd, int stage, const R* __res
         for (int v = 0; v < 5; ++v) P[v] = Psub[v * b.nc + c];
         int pf = 0, ff = 0;
         double rf, uf;
-        geom_floors<GEO>(cst, gd, j, i, rf, uf);
-        with_center_geom<GEO>(gd, j, i, [&](const auto& g) {
+        geom_floors<0>(cst, gd, j, i, rf, uf);
+        with_center_geom<0>(gd, j, i, [&](const auto& g) {
             pf = invert_zone<INV>(g, U, P, cst);
             const int ff0 = (pf / F_GEOM_RHO) * F_GEOM_RHO;
             pf = pf % F_GEOM_RHO;
@@ -145,7 +133,7 @@ extern template void launch_update_geo<double>(
     const BlockDims&, const StepConsts&, const GeomDev&, int, bool, const void*, const void*, const double*,
     const double*, const double*, double*, double*, float*, int*, int*, int*, DeviceState*, double*, hipStream_t,
     double*, const Pack*);
-template <typename R, int GEO, bool PK>
+template <typename R, bool PK>
 static void launch_update_t_k(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int stage, bool do_dt,
                             const void* F, const void* ctop, const double* Usub, const double* Ufull, const double* Psub,
                             double* Uout, double* Pout, float* Pout32, int* pflag, int* fflag,
@@ -156,7 +144,7 @@ static void launch_update_t_k(const BlockDims& b, const StepConsts& c, const Geo
     const BlockEntry* pd = pack_dev(pk);
     constexpr int ND3 = sizeof(R) == 4 ? 3 : 0;
 #define KH_UPD(DT, ND, BM, INV)                                                                                         \
-    hipLaunchKernelGGL((update_kernel<R, DT, ND, BM, GEO, INV, PK>), g, dim3(BS), 0, s, b, c, gd, stage, (const R*)F, (const R*)ctop, \
+    hipLaunchKernelGGL((update_kernel<R, DT, ND, BM, INV, PK>), g, dim3(BS), 0, s, b, c, gd, stage, (const R*)F, (const R*)ctop, \
                        Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, fB, pd)
 #define KH_UPD_BM(DT, INV)                                                                                            \
     {                                                                                                                 \
@@ -173,15 +161,15 @@ static void launch_update_t_k(const BlockDims& b, const StepConsts& c, const Geo
 #undef KH_UPD_BM
 #undef KH_UPD
 }
-template <typename R, int GEO>
+template <typename R>
 static void launch_update_t(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int stage, bool do_dt,
                             const void* F, const void* ctop, const double* Usub, const double* Ufull, const double* Psub,
                             double* Uout, double* Pout, float* Pout32, int* pflag, int* fflag,
                             int* fail_list, DeviceState* ds, double* dt_part, hipStream_t s, const double* fB = nullptr,
                             const Pack* pk = nullptr) {
-    if (pk) launch_update_t_k<R, GEO, true>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32,
+    if (pk) launch_update_t_k<R, true>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32,
                                             pflag, fflag, fail_list, ds, dt_part, s, fB, pk);
-    else launch_update_t_k<R, GEO, false>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32,
+    else launch_update_t_k<R, false>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32,
                                           pflag, fflag, fail_list, ds, dt_part, s, fB, pk);
 }
 hipError_t launch_update_faces(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int prec, int stage,
@@ -190,10 +178,10 @@ hipError_t launch_update_faces(const BlockDims& b, const StepConsts& c, const Ge
                                int* fail_list, DeviceState* ds, double* dt_part, const double* fB, hipStream_t s) {
     if (b.geo || !fB) return hipErrorInvalidValue;
     if (prec == PREC_SPLIT)
-        launch_update_t<float, 0>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag,
+        launch_update_t<float>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag,
                                   fail_list, ds, dt_part, s, fB);
     else
-        launch_update_t<double, 0>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag,
+        launch_update_t<double>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag,
                                    fail_list, ds, dt_part, s, fB);
     return hipGetLastError();
 }
@@ -203,10 +191,10 @@ hipError_t launch_update(const BlockDims& b, const StepConsts& c, const GeomDev&
                          int* fail_list, DeviceState* ds, double* dt_part, hipStream_t s, const Pack* pk) {
     if (prec == PREC_SPLIT) {
         if (b.geo) launch_update_geo<float>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, nullptr, pk);
-        else launch_update_t<float, 0>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, nullptr, pk);
+        else launch_update_t<float>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, nullptr, pk);
     } else {
         if (b.geo) launch_update_geo<double>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, nullptr, pk);
-        else launch_update_t<double, 0>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, nullptr, pk);
+        else launch_update_t<double>(b, c, gd, stage, do_dt, F, ctop, Usub, Ufull, Psub, Uout, Pout, Pout32, pflag, fflag, fail_list, ds, dt_part, s, nullptr, pk);
     }
     return hipGetLastError();
 }
