@@ -78,7 +78,7 @@ int recompute_stage(kh_adjoint* a, int stage) {
     int* fflag = a->floors ? a->ffs[stage - 1] : d->fflag;
     double* F = (double*)d->F;
     double* ct = (double*)d->ctop;
-    KA_HIP(launch_flux_stage_all(bd, c, b->geo, b->p.recon, b->p.precision, SPEEDS_NONE, Psub, nullptr, F, ct, s));
+    KA_HIP(launch_flux_stage_all(bd, c, b->geo, b->route, b->p.recon, b->p.precision, SPEEDS_NONE, Psub, nullptr, F, ct, s));
     if (a->physical) {
         KA_HIP(launch_fix_flux(bd, b->p.precision, F, s));
         KA_HIP(launch_save_x1_flux(bd, F, a->x1f[stage - 1], s));

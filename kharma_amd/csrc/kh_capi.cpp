@@ -114,7 +114,6 @@ void kh::make_dims(const kh_params* p, BlockDims& b) {
     b.ndim = (p->nx3 > 1) ? 3 : ((p->nx2 > 1) ? 2 : 1);
     b.ng = p->ng;
     b.nx1 = p->nx1; b.nx2 = p->nx2; b.nx3 = p->nx3;
-    b.mesh_nx[0] = p->nx1; b.mesh_nx[1] = p->nx2; b.mesh_nx[2] = p->nx3;
     b.n1 = p->nx1 + 2 * p->ng;
     b.n2 = (b.ndim > 1) ? p->nx2 + 2 * p->ng : 1;
     b.n3 = (b.ndim > 2) ? p->nx3 + 2 * p->ng : 1;
@@ -187,8 +186,9 @@ void fill_consts(const kh_params* p, StepConsts& c) {
 // Build the block's metric cache on the host and copy it to the device: FP64
 // tables for the centre and the X1/X2 faces (the flux kernels of the split form
 // read FP32 copies), sqrt(-g) Gamma at centres with a mask of its non-zero
-// components, and the geometric floors.
-hipError_t upload_geometry(kh_block* b) {
+// components, and the geometric floors.  lane_form: g_{t x2} and g_{x2 phi} are
+// zero at every point.
+hipError_t upload_geometry(kh_block* b, bool& lane_form) {
     GeomHost G;
     build_geometry(b->p, b->dims, G);
     GeomDev& d = b->geo;
@@ -211,10 +211,10 @@ hipError_t upload_geometry(kh_block* b) {
         if (e != hipSuccess) return e;
         d.g32[loc] = (const float*)q;
     }
-    d.lane_form = true;
+    lane_form = true;
     for (int loc = 0; loc < 3; ++loc)
         for (int comp : {2, 8})
-            for (long q = 0; q < G.np; ++q) d.lane_form &= G.g[loc][(size_t)comp * G.np + q] == 0.;
+            for (long q = 0; q < G.np; ++q) lane_form &= G.g[loc][(size_t)comp * G.np + q] == 0.;
     unsigned long long mask = 0;
     for (int n = 0; n < 64; ++n)
         for (long q = 0; q < G.np; ++q)
@@ -315,7 +315,9 @@ int kh_block_create(const kh_params* p, kh_block** out) {
     b->npartials = std::max(update_blocks(b->dims), divb_blocks(b->dims)) + 1;
     hipError_t e = hipMalloc(&b->scratch, sizeof(DeviceState));
     if (e == hipSuccess) e = hipMalloc(&b->partials, sizeof(double) * b->npartials);
-    if (e == hipSuccess && b->dims.geo) e = upload_geometry(b);
+    bool lane_form = false;
+    if (e == hipSuccess && b->dims.geo) e = upload_geometry(b, lane_form);
+    b->route = flux_route(b->dims, (long)p->nx1 * p->nx2 * p->nx3, lane_form);
     if (e == hipSuccess) e = upload_fofc_fixed(b);
     if (e == hipSuccess && b->dims.face_ct) e = hipMalloc(&b->ct_cemf, sizeof(double) * 3 * b->dims.nc);
     if (e != hipSuccess) {
@@ -346,7 +348,6 @@ int kh::block_create_in_mesh(const kh_params* mesh, const int nb[3], const int b
     b->p = pb;
     BlockDims& bd = b->dims;
     fill_dims(&pb, bd);
-    bd.mesh_nx[0] = mesh->nx1; bd.mesh_nx[1] = mesh->nx2; bd.mesh_nx[2] = mesh->nx3;
     bd.dx1 = (mesh->x1max - mesh->x1min) / mesh->nx1;
     bd.dx2 = (mesh->x2max - mesh->x2min) / mesh->nx2;
     bd.dx3 = (mesh->x3max - mesh->x3min) / mesh->nx3;
@@ -377,7 +378,9 @@ int kh::block_create_in_mesh(const kh_params* mesh, const int nb[3], const int b
     b->npartials = std::max(update_blocks(bd), divb_blocks(bd)) + 1;
     hipError_t e = hipMalloc(&b->scratch, sizeof(DeviceState));
     if (e == hipSuccess) e = hipMalloc(&b->partials, sizeof(double) * b->npartials);
-    if (e == hipSuccess && bd.geo) e = upload_geometry(b);
+    bool lane_form = false;
+    if (e == hipSuccess && bd.geo) e = upload_geometry(b, lane_form);
+    b->route = flux_route(bd, (long)mesh->nx1 * mesh->nx2 * mesh->nx3, lane_form);
     if (e == hipSuccess) e = upload_fofc_fixed(b);
     if (e != hipSuccess) {
         kh_block_destroy(b);
@@ -431,7 +434,7 @@ int kh_vars_from_pack(void* const* pack_var, int nvar, const kh_varmap* m, kh_va
 int kh_get_flux_v(kh_block* b, int dir, const kh_vars* P, const kh_vars* F_dir, void* cmax_dir, void* cmin_dir) {
     if (!b || !vars_ok(P) || !vars_ok(F_dir) || !cmax_dir || !cmin_dir) return fail(KH_ERR_INVALID, "null argument");
     if (dir < 1 || dir > 3) return fail(KH_ERR_INVALID, "dir must be 1, 2 or 3");
-    KH_HIP(launch_flux(b->dims, b->consts, b->geo, dir, b->p.recon, b->p.precision, vars_in<const double>(P),
+    KH_HIP(launch_flux(b->dims, b->consts, b->geo, b->route, dir, b->p.recon, b->p.precision, vars_in<const double>(P),
                        vars_in<void>(F_dir), cmax_dir, cmin_dir, b->stream));
     return KH_OK;
 }
@@ -1000,9 +1003,9 @@ int kh::driver_stage(kh_driver* d, int stage) {
     // signal speeds only feed the timestep estimate of the last stage
     const int speeds = (stage == 2) ? SPEEDS_CTOP : SPEEDS_NONE;
     if (!d->timing)
-        KH_HIP(launch_flux_stage_all(bd, c, b->geo, b->p.recon, prec, speeds, Psub, Psubf, F, ct, s));
+        KH_HIP(launch_flux_stage_all(bd, c, b->geo, b->route, b->p.recon, prec, speeds, Psub, Psubf, F, ct, s));
     else for (int dir = 1; dir <= bd.ndim; ++dir)   // timed by direction
-        KH_TIMED(dir - 1, launch_flux_stage(bd, c, b->geo, dir, b->p.recon, prec, speeds, Psub, Psubf,
+        KH_TIMED(dir - 1, launch_flux_stage(bd, c, b->geo, b->route, dir, b->p.recon, prec, speeds, Psub, Psubf,
                                             F + fe * (dir - 1) * NV * bd.nc, ct + fe * (dir - 1) * bd.nc, s));
     if (b->p.fofc) {
         // KHARMADriver::AddFOFC (kharma_step.cpp:168-173): on the raw fluxes, before the flux fixes

@@ -519,12 +519,11 @@ flux_x1_march_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const double> P
 // 192x128x128 210 / 180; X1 flat 128^3 112 / 118 (four wavefronts of 103 registers: the
 // tiles stay).  (2-D blocks have one row of each along x3 and too few faces: tiles.)
 constexpr long MARCH_LANES = 2L * 4 * 256 * 64;
-static long mesh_zones(const BlockDims& b) { return (long)b.mesh_nx[0] * b.mesh_nx[1] * b.mesh_nx[2]; }
-static bool march_xt(const BlockDims& b, const GeomDev& gd) {
-    return b.ndim == 3 && (b.geo ? gd.lane_form && mesh_zones(b) >= 5 * MARCH_LANES : mesh_zones(b) >= 7 * MARCH_LANES);
-}
-static bool march_x1(const BlockDims& b, const GeomDev& gd) {
-    return b.geo && gd.lane_form && b.ndim == 3 && mesh_zones(b) >= 8 * MARCH_LANES;
+FluxRoute flux_route(const BlockDims& b, long mesh_zones, bool lane_form) {
+    FluxRoute rt;
+    rt.xt = b.ndim == 3 && (b.geo ? lane_form && mesh_zones >= 5 * MARCH_LANES : mesh_zones >= 7 * MARCH_LANES);
+    rt.x1 = rt.xt && b.geo && mesh_zones >= 8 * MARCH_LANES;
+    return rt;
 }
 // Faces per chunk: the fewest rounds of work for the busiest CU, a round being one
 // block's chunk plus its start, 0.6 of a row's work (flat 160^3, X2: chunks of 1, 2, 4, 22
@@ -544,7 +543,7 @@ static int march_chunk(long blocks_x, int nfaces) {
 }
 
 template <int RECON, int SPEEDS, typename R, typename PT, int GEO, bool PK>
-static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, const Vars<const PT>& P, const Vars<R>& F,
+static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int dir, const Vars<const PT>& P, const Vars<R>& F,
                                R* cmax, R* cmin, hipStream_t s, const Pack* pk) {
     const BlockEntry* pd = pack_dev(pk);
     // Face ranges consumed by flux-CT and the divergence: the face-normal index
@@ -556,7 +555,7 @@ static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const Ge
         if (dir == 1) {
             const int nj = jhi - jlo + 1, nk = khi - klo + 1;
             const long cells = (long)(b.nx1 + 6) * nj;
-            if (march_x1(b, gd)) {
+            if (rt.x1) {
                 const unsigned bx = (unsigned)((cells + 4 * 63 - 1) / (4 * 63));
                 const int chunk = march_chunk((long)bx * nblk, nk);
                 const dim3 grid = pack_grid(dim3(bx, (unsigned)((nk + chunk - 1) / chunk)), pk);
@@ -568,7 +567,7 @@ static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const Ge
             const int s0 = dir == 2 ? b.js : b.ks, s1 = dir == 2 ? b.je + 1 : b.ke + 1;
             const long cols = (long)(b.nx1 + 2) * no;
             const int nfaces = s1 - s0 + 1;
-            if (march_xt(b, gd)) {
+            if (rt.xt) {
                 const unsigned bx = (unsigned)((cols + 255) / 256);
                 const int chunk = march_chunk((long)bx * nblk, nfaces);
                 const dim3 grid = pack_grid(dim3(bx, (unsigned)((nfaces + chunk - 1) / chunk)), pk);
@@ -604,60 +603,60 @@ static hipError_t launch_recon(const BlockDims& b, const StepConsts& c, const Ge
 }
 
 template <int SPEEDS, typename R, typename PT, int GEO, bool PK>
-static hipError_t launch_speeds(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, int recon, const Vars<const PT>& P, const Vars<R>& F,
+static hipError_t launch_speeds(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int dir, int recon, const Vars<const PT>& P, const Vars<R>& F,
                                 R* cmax, R* cmin, hipStream_t s, const Pack* pk) {
     switch (recon) {
-    case RECON_DONOR: return launch_recon<RECON_DONOR, SPEEDS, R, PT, GEO, PK>(b, c, gd, dir, P, F, cmax, cmin, s, pk);
-    case RECON_LINEAR_MC: return launch_recon<RECON_LINEAR_MC, SPEEDS, R, PT, GEO, PK>(b, c, gd, dir, P, F, cmax, cmin, s, pk);
-    case RECON_PPM: return launch_recon<RECON_PPM, SPEEDS, R, PT, GEO, PK>(b, c, gd, dir, P, F, cmax, cmin, s, pk);
-    default: return launch_recon<RECON_WENO5, SPEEDS, R, PT, GEO, PK>(b, c, gd, dir, P, F, cmax, cmin, s, pk);
+    case RECON_DONOR: return launch_recon<RECON_DONOR, SPEEDS, R, PT, GEO, PK>(b, c, gd, rt, dir, P, F, cmax, cmin, s, pk);
+    case RECON_LINEAR_MC: return launch_recon<RECON_LINEAR_MC, SPEEDS, R, PT, GEO, PK>(b, c, gd, rt, dir, P, F, cmax, cmin, s, pk);
+    case RECON_PPM: return launch_recon<RECON_PPM, SPEEDS, R, PT, GEO, PK>(b, c, gd, rt, dir, P, F, cmax, cmin, s, pk);
+    default: return launch_recon<RECON_WENO5, SPEEDS, R, PT, GEO, PK>(b, c, gd, rt, dir, P, F, cmax, cmin, s, pk);
     }
 }
 
 template <typename R, typename PT, int GEO, bool PK>
-static hipError_t launch_geo(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, int recon, int speeds,
+static hipError_t launch_geo(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int dir, int recon, int speeds,
                              const Vars<const PT>& P, const Vars<R>& F, R* cmax, R* cmin, hipStream_t s, const Pack* pk) {
-    if (speeds == SPEEDS_CTOP) return launch_speeds<SPEEDS_CTOP, R, PT, GEO, PK>(b, c, gd, dir, recon, P, F, cmax, cmin, s, pk);
-    if (speeds == SPEEDS_NONE) return launch_speeds<SPEEDS_NONE, R, PT, GEO, PK>(b, c, gd, dir, recon, P, F, cmax, cmin, s, pk);
-    if constexpr (!PK) return launch_speeds<SPEEDS_BOTH, R, PT, GEO, PK>(b, c, gd, dir, recon, P, F, cmax, cmin, s, pk);
+    if (speeds == SPEEDS_CTOP) return launch_speeds<SPEEDS_CTOP, R, PT, GEO, PK>(b, c, gd, rt, dir, recon, P, F, cmax, cmin, s, pk);
+    if (speeds == SPEEDS_NONE) return launch_speeds<SPEEDS_NONE, R, PT, GEO, PK>(b, c, gd, rt, dir, recon, P, F, cmax, cmin, s, pk);
+    if constexpr (!PK) return launch_speeds<SPEEDS_BOTH, R, PT, GEO, PK>(b, c, gd, rt, dir, recon, P, F, cmax, cmin, s, pk);
     return hipErrorInvalidValue;   // a pack launch is a stage's: no cmin array
 }
 
 template <typename R, typename PT, bool PK = false>
-static hipError_t launch_prec(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, int recon, int speeds,
+static hipError_t launch_prec(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int dir, int recon, int speeds,
                               const Vars<const PT>& P, const Vars<R>& F, R* cmax, R* cmin, hipStream_t s,
                               const Pack* pk = nullptr) {
-    if (b.geo) return launch_geo<R, PT, 1, PK>(b, c, gd, dir, recon, speeds, P, F, cmax, cmin, s, pk);
-    return launch_geo<R, PT, 0, PK>(b, c, gd, dir, recon, speeds, P, F, cmax, cmin, s, pk);
+    if (b.geo) return launch_geo<R, PT, 1, PK>(b, c, gd, rt, dir, recon, speeds, P, F, cmax, cmin, s, pk);
+    return launch_geo<R, PT, 0, PK>(b, c, gd, rt, dir, recon, speeds, P, F, cmax, cmin, s, pk);
 }
 
-hipError_t launch_flux(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, int recon, int prec,
+hipError_t launch_flux(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int dir, int recon, int prec,
                        const Vars<const double>& P, const Vars<void>& F, void* cmax, void* cmin, hipStream_t s) {
     if (dir == 2 && b.ndim < 2) return hipSuccess;
     if (dir == 3 && b.ndim < 3) return hipSuccess;
     if (prec == PREC_SPLIT)
-        return launch_prec<float, double>(b, c, gd, dir, recon, SPEEDS_BOTH, P, vars_cast<float>(F), (float*)cmax,
+        return launch_prec<float, double>(b, c, gd, rt, dir, recon, SPEEDS_BOTH, P, vars_cast<float>(F), (float*)cmax,
                                           (float*)cmin, s);
-    return launch_prec<double, double>(b, c, gd, dir, recon, SPEEDS_BOTH, P, vars_cast<double>(F), (double*)cmax,
+    return launch_prec<double, double>(b, c, gd, rt, dir, recon, SPEEDS_BOTH, P, vars_cast<double>(F), (double*)cmax,
                                        (double*)cmin, s);
 }
 
-hipError_t launch_flux_stage(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, int recon, int prec,
+hipError_t launch_flux_stage(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int dir, int recon, int prec,
                              int speeds, const double* P, const float* P32, void* F, void* ctop, hipStream_t s,
                              const Pack* pk) {
     if (dir == 2 && b.ndim < 2) return hipSuccess;
     if (dir == 3 && b.ndim < 3) return hipSuccess;
     if (pk) {
         if (prec == PREC_SPLIT)
-            return launch_prec<float, float, true>(b, c, gd, dir, recon, speeds, vars_of(P32, b.nc),
+            return launch_prec<float, float, true>(b, c, gd, rt, dir, recon, speeds, vars_of(P32, b.nc),
                                                    vars_of((float*)F, b.nc), (float*)ctop, nullptr, s, pk);
-        return launch_prec<double, double, true>(b, c, gd, dir, recon, speeds, vars_of(P, b.nc),
+        return launch_prec<double, double, true>(b, c, gd, rt, dir, recon, speeds, vars_of(P, b.nc),
                                                  vars_of((double*)F, b.nc), (double*)ctop, nullptr, s, pk);
     }
     if (prec == PREC_SPLIT)
-        return launch_prec<float, float>(b, c, gd, dir, recon, speeds, vars_of(P32, b.nc), vars_of((float*)F, b.nc),
+        return launch_prec<float, float>(b, c, gd, rt, dir, recon, speeds, vars_of(P32, b.nc), vars_of((float*)F, b.nc),
                                          (float*)ctop, nullptr, s);
-    return launch_prec<double, double>(b, c, gd, dir, recon, speeds, vars_of(P, b.nc), vars_of((double*)F, b.nc),
+    return launch_prec<double, double>(b, c, gd, rt, dir, recon, speeds, vars_of(P, b.nc), vars_of((double*)F, b.nc),
                                        (double*)ctop, nullptr, s);
 }
 
@@ -710,10 +709,10 @@ static hipError_t launch_all_prec(const BlockDims& b, const StepConsts& c, const
     return speeds == SPEEDS_CTOP ? launch_all<SPEEDS_CTOP, R, 0>(b, c, gd, recon, Pv, Fv, ctop, x, n, s)
                                  : launch_all<SPEEDS_NONE, R, 0>(b, c, gd, recon, Pv, Fv, ctop, x, n, s);
 }
-hipError_t launch_flux_stage_all(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int recon, int prec,
+hipError_t launch_flux_stage_all(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int recon, int prec,
                                  int speeds, const double* P, const float* P32, void* F, void* ctop, hipStream_t s) {
     FluxTiles x[3];
-    const bool march = prec == PREC_FP64 && march_xt(b, gd);
+    const bool march = prec == PREC_FP64 && rt.xt;
     const int n = (speeds == SPEEDS_BOTH || march) ? 0 : all_tiles(b, x);
     if (n)
         return prec == PREC_SPLIT
@@ -721,7 +720,7 @@ hipError_t launch_flux_stage_all(const BlockDims& b, const StepConsts& c, const 
                    : launch_all_prec<double>(b, c, gd, recon, speeds, P, (double*)F, (double*)ctop, x, n, s);
     const long e = prec == PREC_SPLIT ? sizeof(float) : sizeof(double);
     for (int dir = 1; dir <= b.ndim; ++dir) {
-        const hipError_t r = launch_flux_stage(b, c, gd, dir, recon, prec, speeds, P, P32, (char*)F + e * (dir - 1) * NV * b.nc,
+        const hipError_t r = launch_flux_stage(b, c, gd, rt, dir, recon, prec, speeds, P, P32, (char*)F + e * (dir - 1) * NV * b.nc,
                                                (char*)ctop + e * (dir - 1) * b.nc, s, nullptr);
         if (r != hipSuccess) return r;
     }

@@ -11,6 +11,7 @@ struct kh_block {
     kh::BlockDims dims;
     kh::StepConsts consts;
     kh::GeomDev geo;                     // device geometry cache (curvilinear metrics only)
+    kh::FluxRoute route;
     std::vector<void*> geo_bufs;     // owned device allocations behind geo
     hipStream_t stream = nullptr;
     kh::DeviceState* scratch = nullptr;  // reductions of the task-level entry points

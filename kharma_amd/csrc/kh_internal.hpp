@@ -42,7 +42,6 @@ struct BlockDims {
     // Interior offset of this block in the mesh (zones per axis); coordinates are
     // x = xmin(mesh) + (i - is + goff + 1/2) dx with the mesh's dx.
     int goff[3];
-    int mesh_nx[3];        // interior zones of the whole mesh (the block's own where it is the mesh)
     // Face-centred constrained transport (B_CT): face and edge arrays are
     // [3][n3+1][n2+1][n1+1], index (k fs3 + j fs2 + i) for the lower face / edge of
     // cell (k, j, i), component stride nf.
@@ -160,7 +159,6 @@ struct GeomDev {
     const float* flr32 = nullptr;
     int gn1 = 0;
     long np = 0;
-    bool lane_form = false;   // g_{t x2} and g_{x2 phi} are zero at every point (mesh: of every block)
 };
 enum SpeedsOut { SPEEDS_NONE = 0, SPEEDS_BOTH = 1, SPEEDS_CTOP = 2 };
 
@@ -213,20 +211,25 @@ void pack_set_sizes(Pack& pk, const BlockDims* dims, int nblk);
 inline const BlockEntry* pack_dev(const Pack* pk) { return pk ? pk->dev : nullptr; }
 
 // ---- launchers (kh_flux.hip) ----
+// Which FP64 flux kernels a block's launches take: marching ones for X2 / X3 and for X1
+// faces, or tiles.  Follows from the whole mesh that the block belongs to, `mesh_zones`
+// interior zones, and from its tables: lane_form, no g_{t x2} nor g_{x2 phi} in them.
+struct FluxRoute { bool xt = false, x1 = false; };
+FluxRoute flux_route(const BlockDims& b, long mesh_zones, bool lane_form);
 // Face fluxes through the faces normal to `dir` that the step consumes:
 // X1 faces i in [is, ie+1], j in [js-1, je+1], k in [ks-1, ke+1] (collapsed in
 // inactive dimensions), cyclically for X2/X3.  F/cmax/cmin point at this
 // direction's arrays ([8][nc] and [nc]); element type float when prec == PREC_SPLIT.
-hipError_t launch_flux(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, int recon, int prec,
+hipError_t launch_flux(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int dir, int recon, int prec,
                        const Vars<const double>& P, const Vars<void>& F, void* cmax, void* cmin, hipStream_t s);
 // Stage-driver variant: speeds = SPEEDS_NONE or SPEEDS_CTOP (ctop = max(cmax, cmin)
 // into ctop[dir-1]); the split form reads the FP32 shadow P32 of the primitives.
-hipError_t launch_flux_stage(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int dir, int recon, int prec,
+hipError_t launch_flux_stage(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int dir, int recon, int prec,
                              int speeds, const double* P, const float* P32, void* F, void* ctop, hipStream_t s,
                              const Pack* pk = nullptr);
 // The same for every direction: F [3][8][nc] and ctop [3][nc], in one launch for a
 // small block.
-hipError_t launch_flux_stage_all(const BlockDims& b, const StepConsts& c, const GeomDev& gd, int recon, int prec,
+hipError_t launch_flux_stage_all(const BlockDims& b, const StepConsts& c, const GeomDev& gd, FluxRoute rt, int recon, int prec,
                                  int speeds, const double* P, const float* P32, void* F, void* ctop, hipStream_t s);
 
 // ---- launchers (kh_step.hip) ----

@@ -6,8 +6,8 @@ namespace kh {
 
 // Slots of one lane: the metric components that the flux through a face normal to
 // DIR needs, then the floors.  g_{t x2} and g_{x2 phi} have none: they vanish in
-// every embedding the cache is built for (GeomDev::lane_form says so of the
-// uploaded tables, and without it the marching kernels are not used).
+// every embedding the cache is built for (the upload checks the tables, and a block
+// whose tables hold others is routed to the tiles: flux_route).
 enum {
     MG_G00, MG_G01, MG_G03, MG_G11, MG_G12, MG_G13, MG_G22, MG_G33, MG_U00, MG_U01, MG_U02, MG_U03, MG_UDD, MG_GDET,
     MG_ALPHA, MG_RF, MG_UF, MG_N

@@ -103,7 +103,7 @@ int mesh_stage(kh_mesh* m, int stage, hipStream_t s) {
         const kh_block* k = m->blk[0];
         const Pack* pk = &m->pack;
         for (int dir = 1; dir <= k->dims.ndim; ++dir)
-            KM_HIP(launch_flux_stage(k->dims, k->consts, k->geo, dir, k->p.recon, prec, speeds, Psub, Psubf,
+            KM_HIP(launch_flux_stage(k->dims, k->consts, k->geo, k->route, dir, k->p.recon, prec, speeds, Psub, Psubf,
                                      F(0) + fe * (dir - 1) * st, ct(0) + fe * (dir - 1) * nc, s, pk));
         if (const int r = fofc(); r != KH_OK) return r;
         if (pk->fix_flux_n) KM_HIP(launch_fix_flux(k->dims, prec, F(0), s, pk));
@@ -118,7 +118,7 @@ int mesh_stage(kh_mesh* m, int stage, hipStream_t s) {
     for (int b = 0; b < md.nblk; ++b) {
         const kh_block* k = m->blk[b];
         for (int dir = 1; dir <= k->dims.ndim; ++dir)
-            KM_HIP(launch_flux_stage(k->dims, k->consts, k->geo, dir, k->p.recon, prec, speeds, Psub + st * b,
+            KM_HIP(launch_flux_stage(k->dims, k->consts, k->geo, k->route, dir, k->p.recon, prec, speeds, Psub + st * b,
                                      f32(Psubf, b), F(b) + fe * (dir - 1) * st, ct(b) + fe * (dir - 1) * nc, s));
     }
     if (const int r = fofc(); r != KH_OK) return r;
@@ -240,9 +240,9 @@ int kh_mesh_create(const kh_params* p, int nb1, int nb2, int nb3, kh_mesh** out)
             k->geo_bufs.clear();
             k->geo = m->blk[b % (nb1 * nb2)]->geo;
         }
-    bool lane_form = true;   // one answer for the mesh: its blocks run the same kernels
-    for (const kh_block* k : m->blk) lane_form &= k->geo.lane_form;
-    for (kh_block* k : m->blk) k->geo.lane_form = lane_form;
+    FluxRoute route = m->blk[0]->route;   // one for the mesh: its blocks run the same kernels
+    for (const kh_block* k : m->blk) route = {route.xt && k->route.xt, route.x1 && k->route.x1};
+    for (kh_block* k : m->blk) k->route = route;
     const BlockDims& bd = m->blk[0]->dims;
     m->n_dt = dt_blocks(bd);
     m->n_divb = divb_blocks(bd);
