@@ -111,8 +111,8 @@ template <typename R, bool A32 = false> struct CachedGeom {
     // recursion: as sym(b, a) for a > b it was not folded after unrolling, and every
     // transposed component cost a scalar loop, a 64-bit multiply and a load of its
     // own (12 of the 32 metric loads of the pair of lower()s in calc_4vecs).  Folded,
-    // both orders share one load: FP64 X2 faces of the 192x128x128 torus 275 -> 234
-    // us, X1 230 -> 192 us, recovery 228 -> 209 us.
+    // both orders share one load: FP64 X2 face tiles of the 192x128x128 torus 275 ->
+    // 234 us, X1 230 -> 192 us.
     static __device__ __forceinline__ constexpr int sym(int a, int b) {
         const int l = a < b ? a : b, h = a < b ? b : a;
         return l == 0 ? h : l == 1 ? 3 + h : l == 2 ? 5 + h : 9;

@@ -14,6 +14,9 @@
 // X2/X3: 64 x TY blocks; x is a flattened transverse index with x1 fastest (so
 // a wavefront reads 64 consecutive values), y walks TY cells along the face
 // normal, consecutive tiles overlapping by one cell.
+// Small blocks run the tiles of all directions in one launch (flux_all_kernel);
+// FP64 fluxes of large 3-D meshes are taken by lanes that walk along the normal
+// (flux_march_kernel, flux_x1_march_kernel).
 #include "kh_internal.hpp"
 #include "kh_lane_geom.hpp"
 
@@ -21,7 +24,7 @@ namespace kh {
 
 // The FP32 kernels, which are VALU-bound, address their arrays through 32-bit
 // offsets (at32: 5-6 % fewer VALU instructions, 6-7 % faster X2/X3); the FP64
-// kernels keep 64-bit indices, which measured faster for them (X1 8 %).
+// tile kernels keep 64-bit indices, which measured faster for them (X1 8 %).
 template <typename R> struct A32Of { static constexpr bool value = sizeof(R) == 4; };
 template <bool A32, class T> __device__ __forceinline__ T& at_idx(T* p, long e) {
     if constexpr (A32) return at32(p, (unsigned)e);
@@ -122,11 +125,10 @@ __device__ __forceinline__ void face_flux(const StepConsts& c, const BlockDims& 
 // X1 faces i in [is, ie+1] of rows j in [j0, j0+nj), k in [k0, k0+nk).
 // Cells i in [is-1, ie+1] (L per row); block b handles flattened cells
 // [255 b, 255 b + 256) and emits the faces of all but its first cell.
-// Waves per SIMD the FP32 flux kernels are built for (the second launch bound):
-// 6 for the X2/X3 kernels (68 VGPRs instead of 91: 11-14 % faster on the
-// 192x128x128 torus) and for the X1 kernels (67-68 instead of 90-115).  The
-// FP64 kernels keep their 140-142 VGPRs: a 4-wave bound spills 28-36 bytes per
-// lane and is slower.
+// Waves per SIMD the FP32 flux kernels are built for (the second launch bound): 6,
+// which holds them to 48-69 VGPRs (7-8 waves fit); unbounded they took 90-115 and X2/X3
+// were 11-14 % slower on the 192x128x128 torus.  The FP64 tiles are not bounded: 101-126
+// VGPRs, four waves.
 template <typename R> struct FluxOcc { static constexpr int w = sizeof(R) == 4 ? 6 : 1; };
 template <int RECON, int SPEEDS, typename R, typename PT, int GEO>
 __device__ __forceinline__ void x1_tile(const BlockDims& b, const StepConsts& c, const GeomDev& gd, const Vars<const PT>& P,
@@ -186,9 +188,10 @@ flux_x1_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R> 
 
 // X2 / X3 faces.  Transverse columns: flattened (outer, i) with i in [is-1, ie+1]
 // fastest; outer = k (X2) or j (X3) from o0.  Along the normal: faces s in
-// [s0, s1]; tile y covers cells s0-1+(TY-1)y .. s0-2+TY+(TY-1)y.  64 x 8 blocks, two (FP64, 103-118 VGPRs)
-// or three (FP32, 63) per CU: 64 x 10 and 64 x 16 FP32 blocks measured 24 % and 2 %
-// slower, 64 x 4, 64 x 12 and 64 x 16 FP64 blocks 5, 3 and 4 % (192x128x128 torus).
+// [s0, s1]; tile y covers cells s0-1+(TY-1)y .. s0-2+TY+(TY-1)y.  64 x 8 blocks, two
+// per CU in FP64 (101-118 VGPRs), three or four in FP32 (48-67): 64 x 10 and 64 x 16
+// FP32 blocks measured 24 % and 2 % slower, 64 x 4, 64 x 12 and 64 x 16 FP64 blocks 5, 3
+// and 4 % (192x128x128 torus).
 constexpr int XT_TY = 8;
 template <int DIR, int RECON, int SPEEDS, typename R, typename PT, int GEO, int TY>
 __device__ __forceinline__ void xt_tile(const BlockDims& b, const StepConsts& c, const GeomDev& gd, const Vars<const PT>& P,
@@ -279,10 +282,10 @@ flux_all_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R>
     }
 }
 
-// ---------------------------------------------------- FP64, large 3-D blocks
-// The tile kernels keep four (FP64) wavefronts per SIMD waiting half their life:
-// 40 stencil loads, a barrier, the metric's loads, all in one short pass per face.
-// The marching kernels walk instead.
+// ---------------------------------------------------- FP64, large 3-D meshes
+// The FP64 tiles wait for half of a wavefront's life (four per SIMD): 40 stencil
+// loads, a barrier, the metric's loads, all in one short pass per face.  The
+// marching kernels walk instead.
 //
 // X2 / X3 faces.  Each lane walks its own column of cells
 // along the face normal, over a chunk of faces, with the five cells of the stencil
@@ -293,14 +296,14 @@ flux_all_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const PT> P, Vars<R>
 // and (X2) the next row's metric are requested at the row's start and used a row
 // later, and no other load follows them (loads complete in order, so any later one
 // would wait for both).  The metric of the row sits in the lane's own LDS slots,
-// as do the two face states, which frees the registers the window needs (two
-// waves per SIMD).  Lanes share nothing: there is no barrier.
+// as do the two face states, which frees the registers the window needs (172-240
+// VGPRs on the torus, two waves per SIMD).  Lanes share nothing: there is no barrier.
 //
-// Bound by FP64 issue and its dependent chains: VALU 68 % busy at two wavefronts
-// (45 % for the tiles at three), 24 % fewer instructions a face.  192x128x128 torus:
-// X2 234 -> 165 us, X3 226 -> 144 us.  Asking for the next row before the metric
-// (249 us X2: the metric's waits included the prefetch) and the metric straight
-// from memory behind it (250 us X2, 182 us X3) were slower.
+// Bound by FP64 issue and its dependent chains at two wavefronts: VALU issue 0.56-0.63
+// of the chip's capacity on the 192x128x128 torus, waiting 0.31-0.37 of a wavefront's
+// life.  Against the tiles there X2 234 -> 157-163 us, X3 226 -> 139 us.  Asking for the next
+// row before the metric (249 us X2: the metric's waits included the prefetch) and the
+// metric straight from memory behind it (250 us X2, 182 us X3) were slower.
 //
 // The marching kernels' reconstruction: WENO5 in its lean form (X2 172 -> 165 us, X3 154 ->
 // 144, X1 171 -> 160 on the 192x128x128 torus), which rounds differently from the tiles'.
@@ -414,7 +417,7 @@ flux_march_kernel(BlockDims b, StepConsts c, GeomDev gd, Vars<const double> P, V
 // cells pass through LDS (one load a cell instead of five, requested a row ahead);
 // the metric, which x3 does not change, is read once.  A wavefront takes 63 faces
 // and shares nothing with the others: the LDS exchange needs no barrier, only that
-// its accesses stay in order.
+// its accesses stay in order.  192x128x128 torus 192 -> 150 us (VALU issue 0.59).
 __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();

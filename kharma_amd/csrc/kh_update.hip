@@ -19,7 +19,8 @@ namespace kh {
 // fluxes are requested in one go instead of in two parts about a branch, which suits
 // 2-D blocks and FP32 fluxes: FP64 256^2 13.4 / 15.9 -> 12.2 / 14.7 us, split 128^3 213 /
 // 270 -> 212 / 257 us (stage 1 / 2).  The 48 FP64 fluxes of a 3-D zone do not fit 128
-// registers at once (168-196 byte spill; at three wavefronts 64^3 29 / 34 -> 32 / 40 us).
+// registers at once (168-196 byte spill; at three wavefronts 64^3 29 / 34 -> 32 / 40 us);
+// in two parts 24-52 bytes spill.
 // BM: 0 no B transport (1-D), 1 flux-CT EMFs from the face fluxes, 2 face-centred
 // B (B_CT): the cell B is the average of the stage's new faces fB (B_CT::BlockUtoP,
 // b_ct.cpp:173-205, which the reference runs before the inversion).

@@ -71,19 +71,25 @@ __device__ __forceinline__ void recover_zone(const BlockDims& b, const StepConst
 // and the first of the two spent its life waiting on loads while the second, bound
 // by FP64 chains, left memory idle.  Fused, the recovery of one wavefront overlaps
 // the loads of another.  192x128x128 torus, stage 1 / stage 2: FP64 551 / 601 ->
-// 411 / 476 us, FP32 fluxes 500 / 536 -> 387 / 449 us; the 2x2x4 mesh of it 572 /
-// 645 -> 487 / 547 us; 256x128, FP64: 18 / 20 -> 13 / 14.5 us.  The bytes that cannot be
-// avoided take 270-330 us at the rate of a copy.
+// 418 / 473 us, FP32 fluxes 500 / 536 -> 383 / 446 us, these as 2x2x4 blocks 572 / 645 ->
+// 494 / 541 us; 256x128, FP64: 18 / 20 -> 13.5 / 14.5 us.  The bytes that cannot be avoided
+// take 270-330 us at the rate of a copy.
 //
 // In 3-D the zones run on tiles with the metric and floors staged in LDS, which
 // both halves read (stage 1 / 2 unstaged 499 / 562 us).  Three wavefronts per SIMD
-// (168 VGPRs; stage 1 takes 126 and runs four): a bound of four spills 28-76
-// bytes and slows stage 2 (482 -> 525 us).  Staging the 40 connection components
-// too measured 455 / 499 us, requesting the primitives ahead of the staging
-// barrier 441 / 487 us.  The source comes before the state and the fluxes are
-// loaded, but for FP64 fluxes in 2-D, whose few wavefronts gain 5 % from requesting
-// the fluxes first; there the halves are also kept apart for the scheduler (15.6 /
-// 17.7 -> 13.4 / 15 us), and the bound is two wavefronts (none of 3 would be filled).
+// (118-168 VGPRs; with FP32 fluxes and onedw stage 1 takes 124-126 in the drift frame
+// and runs four): a bound of four spills 28-76 bytes and slows stage 2 (482 -> 525 us).  Staging
+// the 40 connection components too measured 455 / 499 us, requesting the primitives
+// ahead of the staging barrier 441 / 487 us.
+//
+// The source is summed apart, before the state and the fluxes are loaded, but for FP64
+// fluxes in 2-D (and 1-D), which add it to the divergence, after requesting the fluxes,
+// with the halves kept apart for the scheduler and a bound of two wavefronts.  The two
+// round differently: this form keeps the bits of 2-D FP64 runs and their gradients.
+// In time it holds its own in small blocks only.  Stage 1 / 2 of the 2-D torus in this
+// form against the 3-D one (three wavefronts): 256x128 14.8 / 15.9 and 14.5 / 16.2 us,
+// 512x256 28 / 30 and 26 / 28.5, 1024x512 107 / 116 and 98 / 109, 2048x1536 624 / 699 and
+// 602 / 662.
 //
 // The guess passes through an empty asm: the source and the solver form the same
 // products of it, and sharing them would round the solver's differently from a
